@@ -9,7 +9,7 @@
 
 #include <stdint.h>
 
-#define MTK_KARGS_VERSION 11
+#define MTK_KARGS_VERSION 12
 
 /* In-workgroup split-K: bytes of workspace slot per output tile of BM x BM (256 or 128). Each
  * wavefront keeps these accumulator blocks (32 x 32 fp32, 4 KB) of its running sum in the slot,
@@ -99,6 +99,11 @@ typedef struct {
   float *lse; /* [B][H][S_q] natural-log row log-sum-exp of the scaled scores, or NULL */
   int32_t H_kv; /* K/V heads (divides H): query head h reads K/V head h / (H / H_kv) */
   int32_t D;    /* head dimension */
+  /* key-split kernels (q_blocks: blocks of 32 (query, query head) rows of one K/V head): */
+  int32_t kv_splits; /* workgroups that share the keys of one row block (>= 1) */
+  int32_t part_ld;   /* floats per row of part */
+  float *part;       /* kv_splits > 1: [B * H_kv][q_blocks][kv_splits][32][part_ld] weighted V sums */
+  float *part_ml;    /* ... and per row (exponent offset in log2, sum of weights) */
 } mtk_attn_kargs;
 
 /* Flash-attention backward (all three kernels of the plan take this block). */

@@ -20,6 +20,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -50,6 +51,7 @@ int fail(int status, const char *fmt, ...) {
 constexpr uint64_t kMaxOperandBytes = (1ull << 31) - 256;  // buffer-resource ranges (see device.hpp)
 constexpr int kAutoKStagger = 16;  // in-workgroup split-K: boundary offsets span up to 16 K-tiles
 constexpr int kMaxHeadDim = MTK_ATTN_MAX_HEAD_DIM;  // largest padded head dimension compiled (512)
+constexpr size_t kPartBytes = 16u << 20;  // partial-sum buffer of a context or graph (attention, keys split)
 
 }  // namespace
 
@@ -60,6 +62,35 @@ struct mtk_ctx {
   hipStream_t stream = nullptr;
   std::vector<hipModule_t> modules;
   std::map<std::string, hipFunction_t> functions;
+  // Partial sums of attention plans that split the keys over workgroups. One buffer for the context's
+  // own stream, whose kernels use it one after another; part_mu is held while a plan enqueues its
+  // kernels, so that two threads' kernels do not interleave on it.
+  std::mutex part_mu;
+  void *part = nullptr;
+
+  // That buffer, or NULL when there is none to be had: work goes to an external stream (which this
+  // context cannot order against its own), the stream is being captured (the graph could replay next
+  // to later work) or the allocation fails. The caller holds part_mu.
+  void *part_buffer() {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusActive;
+    if (stream != own_stream || hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
+      return nullptr;
+    if (!part) part = alloc_part();
+    return part;
+  }
+
+  static void *alloc_part() {
+    // relaxed: another thread's stream capture does not make this allocation an error
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+    void *buf = nullptr;
+    if (hipMalloc(&buf, kPartBytes) != hipSuccess) {
+      buf = nullptr;
+      (void)hipGetLastError();
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return buf;
+  }
 
   int function(const std::string &name, hipFunction_t *f) {
     auto it = functions.find(name);
@@ -105,7 +136,12 @@ struct mtk_plan {
   mtk_conv_desc conv{};
   mtk_permute_desc perm{};
   std::vector<Launch> launches;
+  // attention with the keys split over workgroups: `launches` need a partial-sum buffer of the
+  // library's; `plain` is the plan without one (one kernel), run where there is none
+  bool needs_part = false;
+  std::vector<Launch> plain;
   size_t workspace = 0;
+  size_t part_ml_at = 0;              // byte offset of the per-row pairs in the partial-sum buffer
   size_t weight_bytes = 0;            // conv: exact byte extent of w (its workspace copy is rounded up)
   bool serial_split = false;          // GEMM split-K run in-workgroup (C written by the main kernel)
   unsigned align_a = 2, align_b = 2;  // required operand alignments (bytes)
@@ -117,10 +153,11 @@ namespace {
 
 int resolve(mtk_plan *p) {
   if (!p->ctx) return MTK_OK;
-  for (auto &l : p->launches) {
-    int s = p->ctx->function(l.name, &l.fn);
-    if (s != MTK_OK) return s;
-  }
+  for (auto *ls : {&p->launches, &p->plain})
+    for (auto &l : *ls) {
+      int s = p->ctx->function(l.name, &l.fn);
+      if (s != MTK_OK) return s;
+    }
   return MTK_OK;
 }
 
@@ -801,11 +838,83 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   // 412.4 us); 128 (4 wavefronts, two workgroups
   // per CU) otherwise, causal included (config 5 causal, one box: 298.7 us against 305.3 us for the
   // ping-pong kernel, both in the kernels' balanced causal dispatch order).
+  const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
   int rows = d.q_rows;
   if (rows == 0) {
-    const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
     rows = ((d.D == 128 || d.D == 64) && !d.causal && (long long)d.B * d.H * ((d.S_q + 255) / 256) >= cus) ? 256 : 128;
     if (wide) rows = 64;
+  }
+  // Key-split kernels (attention_kv.hip): the wavefronts of a workgroup share the keys of 32 (query,
+  // query head) rows of one K/V head, so these calls no longer leave most of the device idle.
+  const long long units = (long long)d.B * d.H_kv * (((long long)d.S_q * (d.H / d.H_kv) + 31) / 32);
+  const long long blocks = (long long)d.B * d.H * ((d.S_q + 127) / 128);
+  const int key_tiles = (d.S_kv + 31) / 32;
+  // One box, us per call, 128-query kernel -> key-split kernels:
+  //   few queries behind a cache (a 128-query block would be mostly padding, each query head reads the
+  //     cache again): B 8, H 32/8, 1 x 4096, D 128: 105 -> 33; B 1, H 32/8, 1 x 16384: 281 -> 19;
+  //     B 8, H 32/32, 1 x 4096: 125 -> 98 (5.5 TB/s); but 128 x 128, B 16, H 8: 9.3 against 12.1 (4 key
+  //     tiles for 8 wavefronts)
+  //   sequences of at most half a workgroup per CU: B 1, H 8, 1023 x 1023, D 128: 23.5 -> 12.7; 2048 x
+  //     2048: 41 -> 35, causal 42 -> 24; but B 4, H 12, 512 x 512, D 64 (192 blocks): 11.9 against 16.6.
+  //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the
+  //     plan's choice (its kernel-select is fixed for such shapes; 4 x 1000 x 1000: 23 against 11).
+  const bool decode = d.S_q <= 16 ? (key_tiles >= 8 || units <= cus) : (d.S_q <= 64 && units <= cus);
+  const bool few = blocks * 2 <= cus && key_tiles >= 8 && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
+  if (d.q_rows == 0 && !gen && !wide && (decode || few)) {
+    const int full = dp == 64 ? 2 : 4;  // 32-dim output blocks per workgroup, at most
+    const int blocks32 = (d.D + 31) / 32;
+    // fewer output blocks per workgroup while all workgroups still run at once: K is read again from
+    // L2 by each, V once (B 1, H 32/8, 1 x 1024, D 128: 10.7 us with all four, 8.2 us with one)
+    int ndb = full;
+    for (int n : {2, 1})
+      if (n < full && !(dp == 256 && n == 1) && units * ((blocks32 + n - 1) / n) <= cus) ndb = n;
+    // long caches: the keys split over workgroups instead, at least 8 tiles (one per wavefront) each,
+    // the partial sums added by a second kernel (which costs 2-3 us: B 1, H 32/8, 1 x 4096: 21.7 ->
+    // 11.5 us, 1 x 1024: 8.2 against 8.8; more rows write more partials: H 32/8, 17 x 2048, B 2: 13.5
+    // against 15.1, 64 x 4096, B 1: 23 -> 19)
+    const long long wgs = units * ((blocks32 + full - 1) / full);
+    int splits = (int)std::min<long long>(cus / std::max<long long>(wgs, 1), key_tiles / 8);
+    if (splits < 2 || key_tiles < ((long long)d.B * d.H * d.S_q <= 512 ? 48 : 96)) splits = 1;
+    auto kv_launch = [&](int n, int sp) {
+      Launch l;
+      l.name = "mtk_attn_kv_d" + std::to_string(dp) + "_" + std::to_string(n) + (d.dtype == MTK_F16 ? "_f16" : "_bf16");
+      l.block = dp == 256 ? 256 : 512;
+      mtk_attn_kargs a{};
+      a.B = d.B;
+      a.H = d.H;
+      a.H_kv = d.H_kv;
+      a.S_q = d.S_q;
+      a.S_kv = d.S_kv;
+      a.q_blocks = (int)(units / ((long long)d.B * d.H_kv));
+      a.causal = d.causal ? 1 : 0;
+      a.scale_log2 = (float)(1.4426950408889634 / std::sqrt((double)d.D));
+      a.q_bytes = (uint32_t)q_bytes;
+      a.kv_bytes = (uint32_t)kv_bytes;
+      a.D = d.D;
+      a.kv_splits = sp;
+      a.part_ld = (blocks32 + n - 1) / n * n * 32;
+      l.grid = (unsigned)(units * ((blocks32 + n - 1) / n) * sp);
+      set_args(l, a);
+      return l;
+    };
+    // partial sums, then the rows' (exponent offset, weight sum) pairs
+    const size_t part_rows = (size_t)units * splits * 32;
+    const size_t ml_at = part_rows * ((blocks32 + full - 1) / full * full * 32) * sizeof(float);
+    if (ml_at + part_rows * 8 > kPartBytes) splits = 1;
+    if (splits > 1) {
+      p->needs_part = true;
+      p->part_ml_at = ml_at;
+      p->plain.push_back(kv_launch(ndb, 1));
+      p->launches.push_back(kv_launch(full, splits));
+      Launch c = p->launches[0];
+      c.name = std::string("mtk_attn_kv_combine_") + (d.dtype == MTK_F16 ? "f16" : "bf16");
+      c.block = 256;
+      c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 8) + 255) / 256);
+      p->launches.push_back(c);
+    } else {
+      p->launches.push_back(kv_launch(ndb, 1));
+    }
+    rows = 32;
   }
   Launch g;
   std::string family;
@@ -831,7 +940,7 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   a.D = d.D;
   g.grid = (unsigned)((long long)a.q_blocks * d.B * d.H);
   set_args(g, a);
-  p->launches.push_back(g);
+  if (p->launches.empty()) p->launches.push_back(g);
   double pairs = (double)d.S_q * d.S_kv;
   if (d.causal) {  // exact count of unmasked (i, j): j <= i + (S_kv - S_q)
     pairs = 0;
@@ -844,7 +953,7 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   p->bytes = 2.0 * (double)q_bytes + 2.0 * (double)kv_bytes;
   char desc[256];
   snprintf(desc, sizeof desc, "attention fwd %s B=%d H=%d H_kv=%d S_q=%d S_kv=%d D=%d causal=%d rows/wg=%d grid=%u",
-           d.dtype == MTK_F16 ? "f16" : "bf16", d.B, d.H, d.H_kv, d.S_q, d.S_kv, d.D, d.causal, rows, g.grid);
+           d.dtype == MTK_F16 ? "f16" : "bf16", d.B, d.H, d.H_kv, d.S_q, d.S_kv, d.D, d.causal, rows, p->launches[0].grid);
   p->description = desc;
   int s = resolve(p);
   if (s != MTK_OK) {
@@ -895,8 +1004,9 @@ void patch_gemm(const mtk_plan *p, const Launch &l, char *block, const mtk_gemm_
   }
 }
 
-int bind_args(const mtk_plan *p, const void *argset, std::vector<Launch> &ls) {
-  ls = p->launches;
+// part: the partial-sum buffer for a plan that needs one (NULL: bind the plan without it)
+int bind_args(const mtk_plan *p, const void *argset, std::vector<Launch> &ls, void *part = nullptr) {
+  ls = p->needs_part && !part ? p->plain : p->launches;
   if (p->kind == PLAN_GEMM) {
     const mtk_gemm_args *g = (const mtk_gemm_args *)argset;
     int s = check_gemm_args(p, g);
@@ -971,12 +1081,16 @@ int bind_args(const mtk_plan *p, const void *argset, std::vector<Launch> &ls) {
     if (!aligned(t->Q, al) || !aligned(t->K, al) || !aligned(t->V, al) || !aligned(t->O, al))
       return fail(MTK_ERR_INVALID, "Q, K, V, O must be %u-byte aligned for this plan", al);
     if (t->lse && !aligned(t->lse, 4)) return fail(MTK_ERR_INVALID, "lse must be 4-byte aligned");
-    mtk_attn_kargs &a = args_of<mtk_attn_kargs>(ls[0]);
-    a.Q = t->Q;
-    a.K = t->K;
-    a.V = t->V;
-    a.O = t->O;
-    a.lse = t->lse;
+    for (Launch &l : ls) {
+      mtk_attn_kargs &a = args_of<mtk_attn_kargs>(l);
+      a.Q = t->Q;
+      a.K = t->K;
+      a.V = t->V;
+      a.O = t->O;
+      a.lse = t->lse;
+      a.part = (float *)part;
+      a.part_ml = part ? (float *)((char *)part + p->part_ml_at) : nullptr;
+    }
   }
   return MTK_OK;
 }
@@ -999,10 +1113,16 @@ size_t argset_size(const mtk_plan *p) {
 int run_plan(const mtk_plan *p, const void *argset) {
   if (!p) return fail(MTK_ERR_INVALID, "null plan");
   if (!p->ctx) return fail(MTK_ERR_INVALID, "plan was created without a context (dry plan)");
-  std::vector<Launch> ls;
-  int s = bind_args(p, argset, ls);
-  if (s != MTK_OK) return s;
   HIP_TRY(hipSetDevice(p->ctx->device));
+  std::unique_lock<std::mutex> lock(p->ctx->part_mu, std::defer_lock);
+  void *part = nullptr;
+  if (p->needs_part) {
+    lock.lock();
+    part = p->ctx->part_buffer();
+  }
+  std::vector<Launch> ls;
+  int s = bind_args(p, argset, ls, part);
+  if (s != MTK_OK) return s;
   return launch_all(p, ls, nullptr);
 }
 
@@ -1133,6 +1253,7 @@ int mtk_destroy(mtk_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->own_stream);
     (void)hipStreamDestroy(ctx->own_stream);
   }
+  if (ctx->part) (void)hipFree(ctx->part);
   for (hipModule_t m : ctx->modules) (void)hipModuleUnload(m);
   delete ctx;
   return MTK_OK;
@@ -1314,6 +1435,7 @@ struct mtk_graph {
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  void *part = nullptr;  // the graph's own partial-sum buffer (plans that need one)
 };
 
 int mtk_graph_create(const mtk_plan *p, const void *arg_sets, int nsets, int steps, mtk_graph **out) {
@@ -1322,12 +1444,18 @@ int mtk_graph_create(const mtk_plan *p, const void *arg_sets, int nsets, int ste
   if (steps > 100000) return fail(MTK_ERR_INVALID, "steps above 100000");
   *out = nullptr;
   const size_t stride = argset_size(p);
+  HIP_TRY(hipSetDevice(p->ctx->device));
+  struct Part {  // given to the graph at the end, freed on every earlier return
+    void *buf;
+    ~Part() {
+      if (buf) (void)hipFree(buf);
+    }
+  } part{p->needs_part ? mtk_ctx::alloc_part() : nullptr};
   std::vector<std::vector<Launch>> bound((size_t)nsets);
   for (int i = 0; i < nsets; ++i) {
-    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i]);
+    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i], part.buf);
     if (s != MTK_OK) return s;
   }
-  HIP_TRY(hipSetDevice(p->ctx->device));
   hipStream_t st = p->ctx->stream;
   HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   int status = MTK_OK;
@@ -1363,6 +1491,8 @@ int mtk_graph_create(const mtk_plan *p, const void *arg_sets, int nsets, int ste
   g->stream = st;
   g->graph = graph;
   g->exec = exec;
+  g->part = part.buf;
+  part.buf = nullptr;
   *out = g;
   return MTK_OK;
 }
@@ -1378,6 +1508,7 @@ int mtk_graph_destroy(mtk_graph *g) {
   if (!g) return MTK_OK;
   if (g->exec) (void)hipGraphExecDestroy(g->exec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
+  if (g->part) (void)hipFree(g->part);  // waits for the device
   delete g;
   return MTK_OK;
 }
@@ -1389,17 +1520,23 @@ int mtk_profile(const mtk_plan *p, const void *arg_sets, int nsets, int warmup, 
   if (iters > 100000) return fail(MTK_ERR_INVALID, "iters above 100000");
   memset(out, 0, sizeof *out);
   const size_t stride = argset_size(p);
+  HIP_TRY(hipSetDevice(p->ctx->device));
+  std::unique_lock<std::mutex> lock(p->ctx->part_mu, std::defer_lock);
+  void *part = nullptr;
+  if (p->needs_part) {
+    lock.lock();
+    part = p->ctx->part_buffer();
+  }
   std::vector<std::vector<Launch>> bound((size_t)nsets);
   for (int i = 0; i < nsets; ++i) {
-    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i]);
+    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i], part);
     if (s != MTK_OK) return s;
   }
-  HIP_TRY(hipSetDevice(p->ctx->device));
   for (int i = 0; i < warmup; ++i) {
     int s = launch_all(p, bound[(size_t)(i % nsets)], nullptr);
     if (s != MTK_OK) return s;
   }
-  const size_t nk = p->launches.size();
+  const size_t nk = bound[0].size();
   // Events created so far are destroyed on every exit path; a failed query fails the call (never
   // a silent 0 ms).
   std::vector<hipEvent_t> evs;
@@ -1438,7 +1575,7 @@ int mtk_profile(const mtk_plan *p, const void *arg_sets, int nsets, int warmup, 
     out->n_kernels = (int)std::min<size_t>(nk, 4);
     for (size_t k = 0; k < nk && k < 4; ++k) {
       out->kernel_ms[k] = per[k] / iters;
-      snprintf(out->kernel_names[k], sizeof out->kernel_names[k], "%s", p->launches[k].name.c_str());
+      snprintf(out->kernel_names[k], sizeof out->kernel_names[k], "%s", bound[0][k].name.c_str());
     }
   }
   for (auto &e : evs) (void)hipEventDestroy(e);

@@ -188,7 +188,12 @@ int mtk_gemm_run_noalloc(const mtk_plan *plan, const mtk_gemm_args *args);
  * causal != 0 keeps keys j <= i + (S_kv - S_q) for query i (bottom-right aligned).
  * q_rows: query rows per workgroup, 0 = let the plan choose; 128 (4 wavefronts of 32 queries, two
  * workgroups per CU) or 256 (8 wavefronts of 32 queries in two groups that alternate MFMA and
- * softmax blocks, one workgroup per CU; D = 128 or 64 only). Same results bit for bit. */
+ * softmax blocks, one workgroup per CU; D = 128 or 64 only). Same results bit for bit. With 0, calls
+ * with few queries or one short sequence (D % 8 == 0, up to 256) run kernels that split the keys over
+ * wavefronts and, behind a long cache, over workgroups (sums in a fixed order, reproducible, but not
+ * the order of the 128-row kernel). The latter keep partial sums in a 16 MiB buffer of the context,
+ * allocated once, for work on the context's own stream, and in one of the graph's for mtk_graph_*; on
+ * an external stream or inside a caller's stream capture the keys stay in one workgroup. */
 #define MTK_ATTN_MAX_HEAD_DIM 512
 
 typedef struct {
