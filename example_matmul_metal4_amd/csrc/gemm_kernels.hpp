@@ -7,7 +7,7 @@
 //   *_nn_*_d   B [K][N] (config 1 "C = A.B row-major"), direct-to-LDS + transposed LDS reads
 //   *_tt_*_d, *_tn_*_d   A [K][M] (the reference's transpose.left) with B [N][K] / [K][N]
 //   *_s        split-K with the partitions run in sequence by one workgroup per tile
-//   *_v1       2-byte register-staged fallback for odd leading dimensions
+//   *_v1       register-staged kernels for odd leading dimensions (rows at any 2-byte alignment)
 #pragma once
 
 #include "tile_direct.hpp"

@@ -390,6 +390,9 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     // 127.8 us; 64 tiles 144.3 against 95.3 us).
     const long long t256 = (long long)((d.M + 255) / 256) * ((d.N + 255) / 256);
     tile = (t256 * std::max(split, 1) >= 160 && d.M > 128 && d.N > 128) ? 256 : 128;
+    // odd leading dimensions (register-staged): always 128x128, whose two workgroups per CU cover each
+    // other's loads (4095 cubed, f16: 252 us against 566 us on 256x256, one wavefront per SIMD)
+    if (d.lda % 2 != 0 || d.ldb % 2 != 0) tile = 128;
   }
   const int tiles_m = (d.M + tile - 1) / tile, tiles_n = (d.N + tile - 1) / tile;
   const long long tiles = (long long)tiles_m * tiles_n;
@@ -405,7 +408,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   // Operand rows 4-byte aligned (even leading dimensions): the direct-to-LDS pipeline, with B
   // [N][K] read as row fragments or B [K][N] read through transposed LDS loads (16-byte loads
   // need only dword alignment; a K tail that is not a multiple of 8 is loaded element-wise).
-  // Odd leading dimensions: the register-staged kernel with 2-byte loads.
+  // Odd leading dimensions: the register-staged kernel, rows at any 2-byte alignment.
   const bool direct = d.lda % 2 == 0 && d.ldb % 2 == 0;
   p->align_a = p->align_b = direct ? 4 : 2;
 
@@ -490,7 +493,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   snprintf(desc, sizeof desc,
            "gemm %s %s %s M=%d N=%d K=%d tile=%dx%d split_k=%d k_tiles/split=%d k_stagger=%d %s grid=%u%s", dt,
            d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, tile, tile, split, kps,
-           a.k_stagger, direct ? "direct-to-LDS" : "2-byte loads", g.grid,
+           a.k_stagger, direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
            serial ? " (partitions in sequence per tile, summed in the epilogue)" : split > 1 ? " + splitk_reduce" : "");
   p->description = desc;
   int s = resolve(p);

@@ -71,25 +71,63 @@ __device__ __forceinline__ u32x4 load_chunk(rsrc_t r, OffFn off) {
   }
 }
 
+// 8 halves from any even byte offset: the dwords that hold them (16 + 4 bytes) and a shift by half a
+// dword where the offset is odd in halves. Rows of an odd leading dimension start at such offsets.
+// Issue of loads bounds these kernels: with eight 2-byte loads per chunk 1023 cubed, f16, took 66.7
+// us (B [K][N]: 73.2), with these two 31.1 us (33.1); 2047 x 4095 x 2047 222 -> 63 us.
+__device__ __forceinline__ u32x4 load_chunk_any(rsrc_t r, uint32_t off) {
+  const uint32_t lo = off & ~3u, sh = (off & 2u) << 3;
+  const u32x4 w = buf_load16(r, lo);
+  const uint32_t e = buf_load4(r, lo + 16u);
+  return u32x4{__builtin_amdgcn_alignbit(w.y, w.x, sh), __builtin_amdgcn_alignbit(w.z, w.y, sh),
+               __builtin_amdgcn_alignbit(w.w, w.z, sh), __builtin_amdgcn_alignbit(e, w.w, sh)};
+}
+
+// The first n halves of a chunk, the others zero.
+__device__ __forceinline__ u32x4 keep_halves(u32x4 v, int n) {
+  uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int d = 0; d < 4; ++d) w[d] = 2 * d + 1 < n ? w[d] : 2 * d < n ? w[d] & 0xffffu : 0u;
+  return u32x4{w[0], w[1], w[2], w[3]};
+}
+
+// An operand whose rows are only 2-byte aligned may itself start in the middle of a dword: its
+// buffer starts at that dword, and every offset into it has `mis` (0 or 2) added. kOOBAny lies past
+// any such range.
+constexpr uint32_t kOOBAny = 0x80000000u;
+__device__ __forceinline__ rsrc_t make_rsrc_any(const void *p, uint32_t bytes, uint32_t &mis) {
+  mis = (uint32_t)(uintptr_t)p & 2u;
+  return make_rsrc((const char *)p - mis, (bytes + mis + 3u) & ~3u);
+}
+
 // ---------------------------------------------------------------- A / B loaders
 
-// Row-major operand, rows x K (A [M][lda], or B [N][ldb] in the NK layout).
+// Row-major operand, rows x K (A [M][lda], or B [N][ldb] in the NK layout). V = 1: any alignment.
 template <int ROWS, int V>
 struct LoadRows {
   static constexpr int kPer = ROWS / 32;  // 8 chunks per row, 256 threads -> 32 rows per pass
   uint32_t row_off[kPer];
   int chunk;
 
-  __device__ void init(int tid, int row0, int nrows, int ld) {
+  __device__ void init(int tid, int row0, int nrows, int ld, uint32_t mis) {
     chunk = tid & 7;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int row = row0 + (tid >> 3) + 32 * i;
-      row_off[i] = row < nrows ? (uint32_t)row * (uint32_t)ld * 2u : kOOB;
+      row_off[i] = row < nrows ? (uint32_t)row * (uint32_t)ld * 2u + mis : kOOBAny;
     }
   }
   __device__ void load(rsrc_t r, int kt, int K, u32x4 *out) const {
     const int k = kt * kBK + chunk * 8;
+    if constexpr (V == 1) {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) out[i] = load_chunk_any(r, k < K ? row_off[i] + (uint32_t)k * 2u : kOOBAny);
+      if (K - k < 8) {  // the last K-tile: halves past K belong to the next row
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) out[i] = keep_halves(out[i], K - k);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       out[i] = load_chunk<V>(r, [&](int g) {
@@ -106,7 +144,8 @@ struct LoadRows {
 
 // [K][ld] operand (B in the KN layout, conv weights): 8x8 blocks are transposed in registers
 // so LDS holds the tile K-contiguous, [COLS][64], like the row-major operands.
-template <int COLS, int V>
+// ANY: rows of any alignment (2 bytes).
+template <int COLS, int V, bool ANY>
 struct LoadColsT {
   static constexpr int kNB = COLS / 8;
   static constexpr int kBlocks = 8 * kNB;
@@ -123,7 +162,7 @@ struct LoadColsT {
       nb[p] = b % kNB;
     }
   }
-  __device__ void load(rsrc_t r, int kt, int K, int N, int ld, u32x4 *out, int tid) const {
+  __device__ void load(rsrc_t r, int kt, int K, int N, int ld, uint32_t mis, u32x4 *out, int tid) const {
 #pragma unroll
     for (int p = 0; p < kPer; ++p) {
       if (kBlocks % kThreads != 0 && tid + kThreads * p >= kBlocks) continue;
@@ -132,6 +171,10 @@ struct LoadColsT {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int k = kt * kBK + kb[p] * 8 + i;
+        if constexpr (ANY) {  // columns past N (the next row's) only reach outputs that are not stored
+          raw[i] = load_chunk_any(r, (k < K && n < N) ? ((uint32_t)k * (uint32_t)ld + (uint32_t)n) * 2u + mis : kOOBAny);
+          continue;
+        }
         raw[i] = load_chunk<V>(r, [&](int g) {
           const int nn = n + g * V;
           return (k < K && nn < N) ? ((uint32_t)k * (uint32_t)ld + (uint32_t)nn) * 2u : kOOB;
@@ -302,26 +345,30 @@ __device__ __forceinline__ void tile_gemm(const mtk_tile_args &a) {
   const int kt0 = split_first_tile(a, split, t);
   const int kt1 = split_first_tile(a, split + 1, t);
 
-  const rsrc_t ra = make_rsrc(a.A, a.a_bytes);
-  const rsrc_t rb = make_rsrc(a.B, a.b_bytes);
+  // V = 1 GEMM operands have rows of any alignment; a convolution's are at least element-aligned to
+  // its vector width
+  constexpr bool kAny = AKIND == A_MK && VA == 1;
+  uint32_t mis_a = 0, mis_b = 0;
+  const rsrc_t ra = kAny ? make_rsrc_any(a.A, a.a_bytes, mis_a) : make_rsrc(a.A, a.a_bytes);
+  const rsrc_t rb = kAny ? make_rsrc_any(a.B, a.b_bytes, mis_b) : make_rsrc(a.B, a.b_bytes);
 
   typename ASel<AKIND, BM, VA>::T la;
   if constexpr (AKIND == A_MK) {
-    la.init(tid, m0, a.M, a.lda);
+    la.init(tid, m0, a.M, a.lda, mis_a);
   } else {
     la.init(a, tid, m0);
   }
   constexpr int NA = BM / 32;
   u32x4 rga[NA];
 
-  using LB = typename std::conditional<BKIND == B_NK, LoadRows<BN, VB>, LoadColsT<BN, VB>>::type;
+  using LB = typename std::conditional<BKIND == B_NK, LoadRows<BN, VB>, LoadColsT<BN, VB, kAny>>::type;
   LB lb;
   if constexpr (BKIND == B_NK) {
-    lb.init(tid, n0, a.N, a.ldb);
+    lb.init(tid, n0, a.N, a.ldb, mis_b);
   } else {
     lb.init(tid, n0);
   }
-  constexpr int NB = (BKIND == B_NK) ? BN / 32 : LoadColsT<BN, 1>::kPer * 8;
+  constexpr int NB = (BKIND == B_NK) ? BN / 32 : LB::kPer * 8;
   u32x4 rgb[NB];
 
   auto gload = [&](int kt) {
@@ -333,7 +380,7 @@ __device__ __forceinline__ void tile_gemm(const mtk_tile_args &a) {
     if constexpr (BKIND == B_NK) {
       lb.load(rb, kt, a.K, rgb);
     } else {
-      lb.load(rb, kt, a.K, a.N, a.ldb, rgb, tid);
+      lb.load(rb, kt, a.K, a.N, a.ldb, mis_b, rgb, tid);
     }
   };
   auto lstore = [&](int s) {
