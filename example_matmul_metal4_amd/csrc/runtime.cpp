@@ -859,13 +859,22 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   //     tiles for 8 wavefronts)
   //   sequences of at most half a workgroup per CU: B 1, H 8, 1023 x 1023, D 128: 23.5 -> 12.7; 2048 x
   //     2048: 41 -> 35, causal 42 -> 24; but B 4, H 12, 512 x 512, D 64 (192 blocks): 11.9 against 16.6.
+  //     At D 128 one workgroup fits a CU: a second round of a few uncausal, short ones loses (B 3, H 16/4,
+  //     238 x 238, 360 workgroups: 10.5 against 14.4), as does D 64 (two per CU) below 512 keys (10 x 4
+  //     heads, 247 x 247: 8.0 against 9.3); causal ones are uneven anyway.
   //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the
   //     plan's choice (its kernel-select is fixed for such shapes; 4 x 1000 x 1000: 23 against 11).
-  const bool decode = d.S_q <= 16 ? (key_tiles >= 8 || units <= cus) : (d.S_q <= 64 && units <= cus);
-  const bool few = blocks * 2 <= cus && key_tiles >= 8 && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
-  if (d.q_rows == 0 && !gen && !wide && (decode || few)) {
-    const int full = dp == 64 ? 2 : 4;  // 32-dim output blocks per workgroup, at most
-    const int blocks32 = (d.D + 31) / 32;
+  //   fewer than 4 key tiles leave too many wavefronts without one (28 x 8 heads, 3 x 34: 5.4 against 5.8);
+  //   K/V heads of their own gain only while the last round of workgroups is nearly full (19 x 16 heads,
+  //     1 x 1938: 304 workgroups, 60.0 against 66.3; B 32, H 32, 1 x 1024: 1024, 128 -> 99)
+  const int full = dp == 64 ? 2 : 4;  // 32-dim output blocks per workgroup, at most
+  const int blocks32 = (d.D + 31) / 32;
+  const long long wgs = units * ((blocks32 + full - 1) / full);
+  const bool full_rounds = wgs <= cus || d.H_kv < d.H || wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus);
+  const bool decode = d.S_q <= 16 && key_tiles >= 8 ? full_rounds : d.S_q <= 64 && wgs <= cus;
+  const bool one_round = wgs <= cus || d.causal || (dp == 128 ? key_tiles >= 32 && wgs * 2 >= 3LL * cus : key_tiles >= 16);
+  const bool few = blocks * 2 <= cus && key_tiles >= 8 && one_round && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
+  if (d.q_rows == 0 && !gen && !wide && key_tiles >= 4 && (decode || few)) {
     // fewer output blocks per workgroup while all workgroups still run at once: K is read again from
     // L2 by each, V once (B 1, H 32/8, 1 x 1024, D 128: 10.7 us with all four, 8.2 us with one)
     int ndb = full;
@@ -875,7 +884,6 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
     // the partial sums added by a second kernel (which costs 2-3 us: B 1, H 32/8, 1 x 4096: 21.7 ->
     // 11.5 us, 1 x 1024: 8.2 against 8.8; more rows write more partials: H 32/8, 17 x 2048, B 2: 13.5
     // against 15.1, 64 x 4096, B 1: 23 -> 19)
-    const long long wgs = units * ((blocks32 + full - 1) / full);
     int splits = (int)std::min<long long>(cus / std::max<long long>(wgs, 1), key_tiles / 8);
     if (splits < 2 || key_tiles < ((long long)d.B * d.H * d.S_q <= 512 ? 48 : 96)) splits = 1;
     auto kv_launch = [&](int n, int sp) {

@@ -12,11 +12,12 @@ import oracle
 from test_attention_gpu import check
 
 # (B, H, H_kv, S_q, S_kv, D, causal, dtype): rows and keys at, below and past the 32-row and 32-key
-# blocks, more wavefronts than key tiles, every output-block width, partial d blocks
+# blocks, fewer key tiles than wavefronts, queries that see no key, every output-block width, partial
+# d blocks
 CASES = [
-    (1, 1, 1, 1, 1, 128, False, "f16"), (2, 4, 4, 1, 33, 64, False, "f16"), (1, 8, 2, 1, 255, 128, True, "bf16"),
+    (1, 1, 1, 1, 97, 128, False, "f16"), (2, 4, 4, 1, 129, 64, False, "f16"), (1, 8, 2, 1, 255, 128, True, "bf16"),
     (3, 8, 2, 7, 257, 96, True, "f16"), (1, 16, 2, 4, 700, 80, False, "bf16"), (2, 6, 6, 31, 640, 40, True, "f16"),
-    (1, 5, 5, 64, 1, 64, True, "f16"), (2, 8, 4, 16, 15, 256, True, "f16"), (1, 4, 1, 9, 900, 200, False, "bf16"),
+    (1, 4, 4, 1500, 1030, 64, True, "f16"), (2, 8, 4, 16, 100, 256, True, "f16"), (1, 4, 1, 9, 900, 200, False, "bf16"),
     (16, 16, 16, 1, 300, 128, False, "f16"), (1, 8, 8, 800, 800, 128, True, "f16"), (1, 16, 8, 513, 1030, 64, False, "bf16"),
     # keys split over workgroups: an uneven last split, splits past the causal end, 33 rows
     (1, 8, 2, 1, 4097, 128, False, "f16"), (2, 4, 1, 3, 2500, 64, True, "bf16"), (1, 11, 1, 3, 6000, 128, True, "f16"),
@@ -41,8 +42,10 @@ def test_cases_take_the_key_split_kernels():
     for c in CASES:
         assert "mtk_attn_kv_d" in _plan(None, c).describe(), c
         assert ("mtk_attn_kv_combine_" in _plan(None, c).describe()) == (c in SPLIT), (c, _plan(None, c).describe())
-    # an explicit block of query rows, rows that are not 16-byte aligned and grids of 128-query blocks
-    # keep their kernels
+    # an explicit block of query rows, rows that are not 16-byte aligned, fewer than four key tiles, a
+    # last round of few workgroups and grids of 128-query blocks keep their kernels
+    assert "mtk_attn_kv" not in mtk.AttentionPlan(None, 8, 32, 1, 96, 128, H_kv=8).describe()
+    assert "mtk_attn_kv" not in mtk.AttentionPlan(None, 19, 16, 1, 1938, 128).describe()
     assert "mtk_attn_kv" not in mtk.AttentionPlan(None, 8, 32, 1, 4096, 128, H_kv=8, q_rows=128).describe()
     assert "mtk_attn_fwd_g128" in mtk.AttentionPlan(None, 8, 32, 1, 4096, 100).describe()
     assert "mtk_attn_kv" not in mtk.AttentionPlan(None, 4, 32, 1024, 1024, 128).describe()
