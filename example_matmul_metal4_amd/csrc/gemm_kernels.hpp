@@ -10,6 +10,7 @@
 //   *_v1       register-staged kernels for odd leading dimensions (rows at any 2-byte alignment)
 #pragma once
 
+#include "quarter.hpp"
 #include "tile_direct.hpp"
 
 // 256x256 tiles: 8 wavefronts (2 x 4, 128 x 64 each, two per SIMD); 128x128: 4 (2 x 2).
@@ -21,6 +22,13 @@
 #define MTK_TILE_KERNEL(SUFFIX, BM, BN, WM, WN, AK, BKIND, VA, VB)                             \
   extern "C" __global__ void __launch_bounds__(256) MTK_GEMM_NAME(SUFFIX)(const mtk_tile_args a) { \
     mtk::tile_gemm<MTK_GEMM_DT, BM, BN, WM, WN, mtk::AK, mtk::BKIND, VA, VB>(a);                \
+  }
+
+// the four 64x64 quarters of a 128x128 tile as workgroups, K-tiles over 8 wavefronts (two per SIMD)
+#define MTK_QUARTER_KERNEL(SUFFIX, AT, BN, ANY)                                                                 \
+  extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))                  \
+  MTK_GEMM_NAME(SUFFIX)(const mtk_tile_args a) {                                                               \
+    mtk::quarter_gemm<MTK_GEMM_DT, AT, BN, ANY, 8>(a);                                                          \
   }
 
 namespace mtk_gemm_ops {
@@ -51,6 +59,15 @@ MTK_TILE_KERNEL(nt_256x256_v1, 256, 256, 2, 2, A_MK, B_NK, 1, 1)
 MTK_TILE_KERNEL(nt_128x128_v1, 128, 128, 2, 2, A_MK, B_NK, 1, 1)
 MTK_TILE_KERNEL(nn_256x256_v1, 256, 256, 2, 2, A_MK, B_KN, 1, 1)
 MTK_TILE_KERNEL(nn_128x128_v1, 128, 128, 2, 2, A_MK, B_KN, 1, 1)
+
+MTK_QUARTER_KERNEL(nt_128x128_dq, false, false, false)
+MTK_QUARTER_KERNEL(nn_128x128_dq, false, true, false)
+MTK_QUARTER_KERNEL(tt_128x128_dq, true, false, false)
+MTK_QUARTER_KERNEL(tn_128x128_dq, true, true, false)
+MTK_QUARTER_KERNEL(nt_128x128_v1q, false, false, true)
+MTK_QUARTER_KERNEL(nn_128x128_v1q, false, true, true)
+MTK_QUARTER_KERNEL(tt_128x128_v1q, true, false, true)
+MTK_QUARTER_KERNEL(tn_128x128_v1q, true, true, true)
 
 extern "C" __global__ void __launch_bounds__(256) MTK_REDUCE_NAME(const mtk_reduce_args a) {
   mtk::splitk_reduce<MTK_GEMM_DT>(a);

@@ -214,6 +214,38 @@ float bf16_to_f32(uint16_t h) {
 
 // ------------------------------------------------------------------ GEMM planning
 
+// K partitions of a GEMM on quarter tiles (quarter.hpp: 64x64 workgroups whose 8 wavefronts share the
+// K-tiles), or 0 where the 128x128 tiles are expected to be faster. Chosen by expected time, in us,
+// from launches of 40 shapes on one box (kt: K-tiles of 64; about one workgroup of either kind per CU
+// and round at these sizes):
+//   quarter tiles   1.7 + rounds * (2.5 + 0.20 kt / split)        (rows of any alignment: 0.33)
+//   128x128 tiles   3.6 + 0.57 kt / split, up to 256 workgroups   (1.7)
+//   two or more partitions add a second kernel and its partial sums: 3.5 (quarters), 4.5
+// Measured, 128x128 -> quarters, no split: 1024 cubed 13.3 -> 7.5; 1024 x 1024 x 4096 39.0 -> 17.4; 512 x
+// 512 x 1024 10.0 -> 6.9; 256 cubed 5.7 -> 4.9; 1024 x 2048 x 2048 22.4 -> 19.1; but 640 x 3072 x 768 11.9
+// against 12.4, 1536 cubed 18.6 against 27.0. The plan's own split: 256 x 4096 x 4096 20.4 -> 16.6, 64 x
+// 4096 x 14336 36.7 -> 28.6, but 310 x 2160 x 6864 24.6 against 33.4. Odd leading dimensions, no split:
+// 1023 cubed 31.0 -> 10.5, 2047 x 2047 x 4095 112 -> 94.
+int quarter_split(int M, int N, int k_tiles, int split_k, bool direct, int cus) {
+  if (k_tiles < 4) return 0;  // nothing to share out
+  const long long q = (long long)((M + 63) / 64) * ((N + 63) / 64);
+  const long long t = (long long)((M + 127) / 128) * ((N + 127) / 128);
+  const double kq = direct ? 0.20 : 0.33, k128 = direct ? 0.57 : 1.7;
+  if (t > cus) return 0;
+  auto quarters = [&](int s) {
+    const double rounds = (double)((q * s + cus - 1) / cus);
+    return 1.7 + rounds * (2.5 + kq * ((k_tiles + s - 1) / s)) + (s > 1 ? 3.5 : 0.0);
+  };
+  int s128 = 1;  // the split that 128x128 tiles would take
+  if (split_k == 0 && t * 4 < 3LL * cus) s128 = (int)std::min<long long>({cus / t, std::max(1, k_tiles / 4), 16LL});
+  const double tiles = 3.6 + k128 * ((k_tiles + s128 - 1) / s128) + (s128 > 1 ? 4.5 : 0.0);
+  int best = 1;
+  if (split_k == 0)
+    for (int s = 2; s <= 16 && q * s <= cus && k_tiles >= 6 * s; ++s)
+      if (quarters(s) < quarters(best)) best = s;
+  return quarters(best) < tiles ? best : 0;
+}
+
 int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   if (!d_in || !out) return fail(MTK_ERR_INVALID, "null descriptor or output");
   mtk_gemm_desc d = *d_in;
@@ -380,8 +412,25 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     }
   }
 
+  // Operand rows 4-byte aligned (even leading dimensions): the direct-to-LDS pipeline, with B
+  // [N][K] read as row fragments or B [K][N] read through transposed LDS loads (16-byte loads
+  // need only dword alignment; a K tail that is not a multiple of 8 is loaded element-wise).
+  // Odd leading dimensions: the register-staged kernel, rows at any 2-byte alignment.
+  const bool direct = d.lda % 2 == 0 && d.ldb % 2 == 0;
+  p->align_a = p->align_b = direct ? 4 : 2;
+
   int tile = d.tile;
   int split = d.split_k;
+  // Quarter tiles: only where neither a tile, a partition layout nor a schedule is asked for; and for A
+  // [K][M] with odd rows of B always (no other kernel reads them).
+  int quarter = 0;
+  if (tile == 0 && d.split_mode == MTK_SPLIT_AUTO && d.k_stagger == 0 && split <= 1)
+    quarter = quarter_split(d.M, d.N, k_tiles, split, direct, ctx ? ctx->prop.multiProcessorCount : 256);
+  if (d.trans_a && !direct && !quarter && d.split_mode != MTK_SPLIT_SERIAL) quarter = std::max(1, split);
+  if (quarter) {
+    tile = 128;
+    split = quarter;
+  }
   if (tile == 0) {
     // 256x256 tiles when there are enough of them (with the requested split) to fill most of the
     // device, unless M or N fits a 128 tile: a 256 tile would then compute mostly padding. Below
@@ -394,7 +443,8 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     // other's loads (4095 cubed, f16: 252 us against 566 us on 256x256, one wavefront per SIMD)
     if (d.lda % 2 != 0 || d.ldb % 2 != 0) tile = 128;
   }
-  const int tiles_m = (d.M + tile - 1) / tile, tiles_n = (d.N + tile - 1) / tile;
+  const int edge = quarter ? 64 : tile;  // of a workgroup's tile
+  const int tiles_m = (d.M + edge - 1) / edge, tiles_n = (d.N + edge - 1) / edge;
   const long long tiles = (long long)tiles_m * tiles_n;
   if (split == 0) {  // fill about one wave of 256 CUs with split-K when the tile grid is small
     split = 1;
@@ -405,19 +455,12 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   const int kps = (k_tiles + split - 1) / split;
   split = (k_tiles + kps - 1) / kps;  // no empty splits
 
-  // Operand rows 4-byte aligned (even leading dimensions): the direct-to-LDS pipeline, with B
-  // [N][K] read as row fragments or B [K][N] read through transposed LDS loads (16-byte loads
-  // need only dword alignment; a K tail that is not a multiple of 8 is loaded element-wise).
-  // Odd leading dimensions: the register-staged kernel, rows at any 2-byte alignment.
-  const bool direct = d.lda % 2 == 0 && d.ldb % 2 == 0;
-  p->align_a = p->align_b = direct ? 4 : 2;
-
   // Split-K scheduling. In-workgroup ("serial"): one workgroup per tile walks the partitions in
   // sequence and parks split-1 fp32 partition sums per tile; worth it when the tile grid alone
   // fills the device (every CU busy without extra partition workgroups), and it saves the second
   // kernel and 1/split of the partial traffic.
   bool serial = false;
-  if (split > 1) {
+  if (split > 1 && !quarter) {
     const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
     if (d.split_mode == MTK_SPLIT_SERIAL) {
       if (split > 4 || !direct) {
@@ -434,9 +477,10 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   Launch g;
   char name[96];
   // operand letters: A [M][K] 'n' / [K][M] 't', B [N][K] 't' / [K][N] 'n'
-  snprintf(name, sizeof name, "mtk_gemm_%s_%c%c_%dx%d_%s", dt, d.trans_a ? 't' : 'n', d.trans_b ? 't' : 'n', tile, tile,
-           serial ? "s" : direct ? "d" : "v1");
+  snprintf(name, sizeof name, "mtk_gemm_%s_%c%c_%dx%d_%s%s", dt, d.trans_a ? 't' : 'n', d.trans_b ? 't' : 'n', tile,
+           tile, serial ? "s" : direct ? "d" : "v1", quarter ? "q" : "");
   g.name = name;
+  if (quarter) g.block = 512;
   if (tile == 256 && direct) g.block = 512;  // 256x256 direct-to-LDS tiles run 8 wavefronts
   g.grid = (unsigned)(serial ? tiles : tiles * split);
   mtk_tile_args a{};
@@ -493,7 +537,8 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   snprintf(desc, sizeof desc,
            "gemm %s %s %s M=%d N=%d K=%d tile=%dx%d split_k=%d k_tiles/split=%d k_stagger=%d %s grid=%u%s", dt,
            d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, tile, tile, split, kps,
-           a.k_stagger, direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
+           a.k_stagger,
+           quarter ? "64x64 quarters, K-tiles over 8 wavefronts" : direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
            serial ? " (partitions in sequence per tile, summed in the epilogue)" : split > 1 ? " + splitk_reduce" : "");
   p->description = desc;
   int s = resolve(p);
