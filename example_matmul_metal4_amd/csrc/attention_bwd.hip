@@ -145,9 +145,98 @@ __device__ __forceinline__ void attn_bwd_pre(const mtk_attn_bwd_kargs &a) {
   }
 }
 
+// ------------------------------------------------------------------------------------- shared walks
+
+// Steps [i0, i1) of a walk of n steps for workgroup `part` of those that share it (n > 0), and how many
+// do; part >= that count has none.
+__device__ __forceinline__ int walk_part(int n, int cap, int part, int &i0, int &i1) {
+  const int parts = max(1, (n + cap - 1) / cap);
+  const int per = (n + parts - 1) / parts;
+  i0 = min(n, part * per);
+  i1 = min(n, i0 + per);
+  return parts;
+}
+
+// The walks' lengths: query tiles of every head of the group that see key block k0 .. (dK/dV), key
+// tiles that query block q0 .. sees (dQ).
+__device__ __forceinline__ int dkdv_first_tile(const mtk_attn_bwd_kargs &a, int k0) {
+  return a.causal ? max(0, k0 - (a.S_kv - a.S_q)) / kBwdQTile : 0;
+}
+__device__ __forceinline__ int dkdv_per_head(const mtk_attn_bwd_kargs &a, int k0) {
+  return max(0, (a.S_q + kBwdQTile - 1) / kBwdQTile - dkdv_first_tile(a, k0));
+}
+__device__ __forceinline__ int dq_tiles(const mtk_attn_bwd_kargs &a, int q0) {
+  const int kv_end = a.causal ? min(a.S_kv, q0 + kBwdQRows + a.S_kv - a.S_q) : a.S_kv;
+  return kv_end > 0 ? (kv_end + kBwdKTile - 1) / kBwdKTile : 0;
+}
+
+// One wavefront's 32 rows x 32 NB dims of fp32 sums (accumulator column = row) to rows of D floats at
+// dst (row r: dst + r * ld), through its own LDS region (16-byte chunk c of row r at c ^ (r & 15) or
+// (r & 7)) so that every store instruction writes whole row pieces.
+template <int NB>
+__device__ __forceinline__ void store_part(const f32x16 *acc, char *lds, float *dst, size_t ld, int rows, int dims, int lane) {
+  constexpr int kC = NB * 8, kX = kC >= 16 ? 15 : 7;  // chunks per row
+  const int g = lane >> 5, col = lane & 31;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int db = 0; db < NB; ++db)
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq)
+      *(f32x4 *)(lds + col * (kC * 16) + (((8 * db + 2 * rq + g) ^ (col & kX)) << 4)) =
+          f32x4{acc[db][4 * rq], acc[db][4 * rq + 1], acc[db][4 * rq + 2], acc[db][4 * rq + 3]};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int it = 0; it < kC / 2; ++it) {
+    const int r = it * (64 / kC) + lane / kC, c = lane % kC;
+    const f32x4 v = *(const f32x4 *)(lds + r * (kC * 16) + ((c ^ (r & kX)) << 4));
+    if (r < rows && 4 * c < dims) *(f32x4 *)(dst + (size_t)r * ld + 4 * c) = v;
+  }
+}
+
+// dK, dV and dQ of the shared walks: partial sums added in part order, rounded once. One thread per 8
+// elements of [dK | dV | dQ]; blocks that one workgroup walked alone are already written.
+template <int DT>
+__device__ __forceinline__ void attn_bwd_sum(const mtk_attn_bwd_kargs &a) {
+  const size_t nkv = (size_t)a.B * a.S_kv * a.H_kv * a.D, nq = (size_t)a.B * a.S_q * a.H * a.D;
+  size_t e = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  const float *src;
+  uint16_t *dst;
+  size_t stride;
+  int parts, i0, i1;
+  if (e < 2 * nkv) {
+    if (a.kv_parts < 2) return;
+    src = a.part_kv + e;
+    stride = 2 * nkv;
+    dst = (uint16_t *)(e < nkv ? a.dK : a.dV);
+    if (e >= nkv) e -= nkv;
+    const int k = (int)(e / ((size_t)a.H_kv * a.D) % a.S_kv);
+    parts = walk_part(a.H / a.H_kv * dkdv_per_head(a, k / kBwdKeys * kBwdKeys), a.kv_cap, 0, i0, i1);
+  } else {
+    e -= 2 * nkv;
+    if (e >= nq || a.q_parts < 2) return;
+    src = a.part_q + e;
+    stride = nq;
+    dst = (uint16_t *)a.dQ;
+    const int q = (int)(e / ((size_t)a.H * a.D) % a.S_q);
+    parts = walk_part(dq_tiles(a, q / kBwdQRows * kBwdQRows), a.q_cap, 0, i0, i1);
+  }
+  if (parts < 2) return;
+  f32x4 x = *(const f32x4 *)src, y = *(const f32x4 *)(src + 4);
+#pragma unroll 4
+  for (int p = 1; p < parts; ++p) {
+    x += *(const f32x4 *)(src + p * stride);
+    y += *(const f32x4 *)(src + p * stride + 4);
+  }
+  *(u32x4 *)(dst + e) = u32x4{pack2<DT>(x.x, x.y), pack2<DT>(x.z, x.w), pack2<DT>(y.x, y.y), pack2<DT>(y.z, y.w)};
+}
+
 // ------------------------------------------------------------------------------------- dK, dV
 
-template <int DT, bool CAUSAL, int DP>
+// SHARED (here and in dQ): the walks may be shared by several workgroups. Kernels of their own: the
+// extra index arithmetic took 0.6-1 us of a 28 us call that shares nothing.
+template <int DT, bool CAUSAL, int DP, bool SHARED>
 __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
   using L = AttnLayout<DP>;
   constexpr int kRowTile = L::kTile, kRowB = L::kRowB, kKs = L::kKs, kDb = L::kDb;
@@ -164,9 +253,16 @@ __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
   const int g = lane >> 5, col = lane & 31;
 
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  int bh = id / a.k_blocks;  // (batch, K/V head)
-  int kb = id - bh * a.k_blocks;
-  if (CAUSAL) causal_order(id, a.k_blocks, a.B * a.H_kv, bh, kb);  // heaviest (first) key blocks first
+  const int nblk = SHARED ? a.k_blocks * a.kv_parts : a.k_blocks;
+  int bh = id / nblk;  // (batch, K/V head)
+  int kb = id - bh * nblk;
+  if (CAUSAL) causal_order(id, nblk, a.B * a.H_kv, bh, kb);  // heaviest (first) key blocks first
+  int part = 0, parts = 1;
+  if constexpr (SHARED) {  // a key block's shares side by side
+    part = kb % a.kv_parts;
+    kb /= a.kv_parts;
+    if (CAUSAL && a.k_blocks <= 64) kb = a.kv_order[kb];
+  }
   const int b = bh / a.H_kv, hk = bh - b * a.H_kv;
   const int group = a.H / a.H_kv;  // query heads hk * group .. hk * group + group - 1
   const int k0 = kb * kBwdKeys;
@@ -198,11 +294,13 @@ __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
   // query tiles that see at least one of this workgroup's keys: t0 .. n_tiles - 1 of each query
   // head of the group, visited head by head (step i: head hk * group + i / per_head, tile
   // t0 + i % per_head)
-  int t0 = 0;
-  if (CAUSAL) t0 = max(0, k0 - diag) / kBwdQTile;
-  const int n_tiles = (a.S_q + kBwdQTile - 1) / kBwdQTile;
-  const int per_head = max(0, n_tiles - t0);
-  const int n_steps = group * per_head;
+  int t0 = dkdv_first_tile(a, k0);
+  int per_head = dkdv_per_head(a, k0);
+  int i_first = 0, n_steps = group * per_head;  // this workgroup's steps: i_first .. n_steps - 1
+  if constexpr (SHARED) {
+    parts = walk_part(n_steps, a.kv_cap, part, i_first, n_steps);
+    if (part >= parts) return;
+  }
 
   // Staging of step i (clamped to the last step: past the end a slot is refilled, never read
   // for a result) into the slots given.
@@ -283,15 +381,15 @@ __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
   };
 
   f32x16 s[2], p[2];
-  if (n_steps > 0) {
-    stage_rows_to(0, 0);
-    stage_tr_to(0, 0);
-    stage_rows_to(1, min(1, n_steps - 1));
+  if (n_steps > i_first) {
+    stage_rows_to(i_first & 1, i_first);
+    stage_tr_to(i_first & 1, i_first);
+    stage_rows_to((i_first + 1) & 1, min(i_first + 1, n_steps - 1));
     wait_vmem();
     __syncthreads();
-    sdp(0, s, p, [](auto) {});
+    sdp(i_first & 1, s, p, [](auto) {});
   }
-  for (int i = 0; i < n_steps; ++i) {
+  for (int i = i_first; i < n_steps; ++i) {
     wait_vmem();
     // rows of step i + 1, transposed tiles and row terms of step i have landed; every wave is done
     // with the rows of step i, the transposed tiles and row terms of step i - 1
@@ -402,6 +500,15 @@ __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
   // before the stages are reused for the output tiles (explicit, not left to the fence's own wait).
   wait_vmem();
   __syncthreads();  // every wave is done reading the last stage
+  if (SHARED && parts > 1) {
+    const size_t nkv = (size_t)a.B * a.S_kv * a.H_kv * a.D, ld = (size_t)a.H_kv * a.D;
+    float *dst = a.part_kv + 2 * nkv * part + (((size_t)b * a.S_kv + k0 + wave * 32) * a.H_kv + hk) * a.D;
+    char *own = smem + wave * (32 * 4 * DP);
+    const int rows = a.S_kv - (k0 + wave * 32);
+    store_part<kDb>(dk, own, dst, ld, rows, a.D, lane);
+    store_part<kDb>(dv, own, dst + nkv, ld, rows, a.D, lane);
+    return;
+  }
   char *pk = smem + wave * (2 * 32 * kRowB), *pv = pk + 32 * kRowB;
 #pragma unroll
   for (int db = 0; db < kDb; ++db)
@@ -433,7 +540,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const mtk_attn_bwd_kargs &a) {
 
 // ------------------------------------------------------------------------------------- dQ
 
-template <int DT, bool CAUSAL, int DP>
+template <int DT, bool CAUSAL, int DP, bool SHARED>
 __device__ __forceinline__ void attn_bwd_dq(const mtk_attn_bwd_kargs &a) {
   using L = AttnLayout<DP>;
   constexpr int kRowTile = L::kTile, kRowB = L::kRowB, kKs = L::kKs, kDb = L::kDb;
@@ -445,11 +552,21 @@ __device__ __forceinline__ void attn_bwd_dq(const mtk_attn_bwd_kargs &a) {
   const int g = lane >> 5, col = lane & 31;
 
   const int id = xcd_remap(blockIdx.x, gridDim.x);
-  int bh = id / a.q_blocks;
-  int qblk = id - bh * a.q_blocks;
-  if (CAUSAL) {  // heaviest (last) query blocks first
-    causal_order(id, a.q_blocks, a.B * a.H, bh, qblk);
-    qblk = a.q_blocks - 1 - qblk;
+  const int nblk = SHARED ? a.q_blocks * a.q_parts : a.q_blocks;
+  int bh = id / nblk;
+  int qblk = id - bh * nblk;
+  if (CAUSAL) causal_order(id, nblk, a.B * a.H, bh, qblk);  // heaviest (last) query blocks first
+  int part = 0, parts = 1;
+  if constexpr (SHARED) {  // a query block's shares side by side
+    part = qblk % a.q_parts;
+    qblk /= a.q_parts;
+    if (CAUSAL && a.q_blocks <= 64) qblk = a.q_order[qblk];
+  }
+  if (CAUSAL) qblk = a.q_blocks - 1 - qblk;
+  int t_first = 0, n_tiles = dq_tiles(a, qblk * kBwdQRows);  // this workgroup's key tiles: t_first .. n_tiles - 1
+  if constexpr (SHARED) {
+    parts = walk_part(n_tiles, a.q_cap, part, t_first, n_tiles);
+    if (part >= parts) return;
   }
   const int b = bh / a.H, h = bh - b * a.H;
   const int hk = h / (a.H / a.H_kv);  // K/V head of query head h
@@ -479,10 +596,6 @@ __device__ __forceinline__ void attn_bwd_dq(const mtk_attn_bwd_kargs &a) {
   const float lse2 = q_ok ? a.Lt[ridx] : 0.0f;   // base-2 lse
   const float dterm = q_ok ? a.Dt[ridx] : 0.0f;  // D * scale
 
-  int kv_end = a.S_kv;
-  if (CAUSAL) kv_end = min(a.S_kv, q0 + kBwdQRows + diag);
-  const int n_tiles = kv_end > 0 ? (kv_end + kBwdKTile - 1) / kBwdKTile : 0;
-
   auto stage = [&](int slot, int t) {
     char *st = smem + slot * 3 * kRowTile;
     const int valid = a.S_kv - t * kBwdKTile;
@@ -497,8 +610,8 @@ __device__ __forceinline__ void attn_bwd_dq(const mtk_attn_bwd_kargs &a) {
 #pragma unroll
   for (int i = 0; i < kDb; ++i) dq[i] = f32x16{};
 
-  if (n_tiles > 0) stage(0, 0);
-  for (int t = 0; t < n_tiles; ++t) {
+  if (n_tiles > t_first) stage(t_first & 1, t_first);
+  for (int t = t_first; t < n_tiles; ++t) {
     wait_vmem();
     __syncthreads();  // tile t is in LDS; everyone is done with tile t-1's slot
     if (t + 1 < n_tiles) stage((t + 1) & 1, t + 1);
@@ -596,6 +709,17 @@ __device__ __forceinline__ void attn_bwd_dq(const mtk_attn_bwd_kargs &a) {
   // LDS as rows of DP elements and stored as whole rows, as in the dK/dV kernel (no loads are in flight
   // here: the loop stages no tile past the last and waits for each tile it staged)
   __syncthreads();  // every wave is done reading the last stage
+  if (SHARED && parts > 1) {  // half of the dims at a time: the stages hold half of all rows
+    constexpr int kHalf = kDb / 2;
+    float *dst = a.part_q + (size_t)part * a.B * a.S_q * a.H * a.D +
+                 (((size_t)b * a.S_q + q0 + wave * 32) * a.H + h) * a.D;
+    char *own = smem + wave * (32 * kHalf * 128);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      store_part<kHalf>(dq + x * kHalf, own, dst + x * kHalf * 32, (size_t)a.H * a.D, a.S_q - (q0 + wave * 32),
+                        a.D - x * kHalf * 32, lane);
+    return;
+  }
   char *pq = smem + wave * (32 * kRowB);
 #pragma unroll
   for (int db = 0; db < kDb; ++db)
@@ -620,14 +744,27 @@ using namespace mtk;
 
 #define BWD_PRE(NAME, DT) \
   extern "C" __global__ void __launch_bounds__(256) NAME(const mtk_attn_bwd_kargs a) { attn_bwd_pre<DT>(a); }
-#define BWD_DKDV(NAME, DT, CAUSAL, DP)                                               \
-  extern "C" __global__ void __launch_bounds__(256) NAME(const mtk_attn_bwd_kargs a) { \
-    attn_bwd_dkdv<DT, CAUSAL, DP>(a);                                                \
+#define BWD_DKDV(NAME, DT, CAUSAL, DP)                                                          \
+  extern "C" __global__ void __launch_bounds__(256) NAME(const mtk_attn_bwd_kargs a) {          \
+    attn_bwd_dkdv<DT, CAUSAL, DP, false>(a);                                                    \
+  }                                                                                             \
+  extern "C" __global__ void __launch_bounds__(256) NAME##_shared(const mtk_attn_bwd_kargs a) { \
+    attn_bwd_dkdv<DT, CAUSAL, DP, true>(a);                                                     \
   }
-#define BWD_DQ(NAME, DT, CAUSAL, DP)                                                 \
-  extern "C" __global__ void __launch_bounds__(512) NAME(const mtk_attn_bwd_kargs a) { \
-    attn_bwd_dq<DT, CAUSAL, DP>(a);                                                  \
+#define BWD_DQ(NAME, DT, CAUSAL, DP)                                                            \
+  extern "C" __global__ void __launch_bounds__(512) NAME(const mtk_attn_bwd_kargs a) {          \
+    attn_bwd_dq<DT, CAUSAL, DP, false>(a);                                                      \
+  }                                                                                             \
+  extern "C" __global__ void __launch_bounds__(512) NAME##_shared(const mtk_attn_bwd_kargs a) { \
+    attn_bwd_dq<DT, CAUSAL, DP, true>(a);                                                       \
   }
+
+extern "C" __global__ void __launch_bounds__(256) mtk_attn_bwd_sum_f16(const mtk_attn_bwd_kargs a) {
+  attn_bwd_sum<DT_F16>(a);
+}
+extern "C" __global__ void __launch_bounds__(256) mtk_attn_bwd_sum_bf16(const mtk_attn_bwd_kargs a) {
+  attn_bwd_sum<DT_BF16>(a);
+}
 
 BWD_PRE(mtk_attn_bwd_pre_f16, DT_F16)
 BWD_PRE(mtk_attn_bwd_pre_bf16, DT_BF16)

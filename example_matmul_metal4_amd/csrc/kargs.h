@@ -9,7 +9,7 @@
 
 #include <stdint.h>
 
-#define MTK_KARGS_VERSION 12
+#define MTK_KARGS_VERSION 13
 
 /* In-workgroup split-K: bytes of workspace slot per output tile of BM x BM (256 or 128). Each
  * wavefront keeps these accumulator blocks (32 x 32 fp32, 4 KB) of its running sum in the slot,
@@ -122,6 +122,13 @@ typedef struct {
   uint32_t q_bytes, kv_bytes;
   float *Lt; /* [B][H][S_q] workspace: lse * log2(e) (base-2 log-sum-exp) */
   int32_t D; /* head dimension: a multiple of 8 up to the kernel's padded head dimension */
+  /* Long walks shared by several workgroups: a key block of n steps (dK/dV: query tiles of the group's
+     heads; dQ: key tiles) takes max(1, ceil(n / cap)) of its `parts` workgroups, which leave fp32
+     partial sums for the last kernel when there are two or more of them. */
+  int32_t kv_cap, kv_parts, q_cap, q_parts;
+  uint8_t kv_order[64], q_order[64]; /* shared, causal, at most 64 blocks: block of each rank, longest share first */
+  float *part_kv; /* [kv_parts][2: dK, dV][B][S_kv][H_kv][D] */
+  float *part_q;  /* [q_parts][B][S_q][H][D] */
 } mtk_attn_bwd_kargs;
 
 /* Convolution weight re-layout OIDHW -> DHWIO (16-bit elements). */

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -141,6 +142,7 @@ struct mtk_plan {
   bool needs_part = false;
   std::vector<Launch> plain;
   size_t workspace = 0;
+  size_t lt_at = 0, part_kv_at = 0, part_q_at = 0;  // attention backward: byte offsets in the workspace
   size_t part_ml_at = 0;              // byte offset of the per-row pairs in the partial-sum buffer
   size_t weight_bytes = 0;            // conv: exact byte extent of w (its workspace copy is rounded up)
   bool serial_split = false;          // GEMM split-K run in-workgroup (C written by the main kernel)
@@ -550,6 +552,56 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   return MTK_OK;
 }
 
+// How the walks of an attention backward kernel are shared out: workgroups per block (at most) and the
+// longest walk of one. walks: the blocks' lengths in steps, every block `count` times; a step takes
+// step_us on a nearly idle device, 1.7 times that with every CU at work (D 128: 2.0 and 3.4 us);
+// elems: fp32 values of one set of partial sums. One workgroup fits a CU; the shares are dispatched
+// longest first, so the last ends about half of the longest share after the average (more than 64
+// blocks, which are not sorted by share: a whole one; uncausal: equal walks, whole rounds). Partial
+// sums are written and read once, at about 4 TB/s.
+struct WalkShare {
+  int cap = INT32_MAX, parts = 1;
+  uint8_t order[64] = {};  // indices into walks, longest share first
+};
+WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal, double step_us, double elems, int cus) {
+  const int longest = *std::max_element(walks.begin(), walks.end());
+  auto expected = [&](int cap) {
+    double total = 0, shared = 0;
+    long long n = 0;
+    int item = 0;
+    for (int w : walks) {
+      const int parts = std::max(1, (w + cap - 1) / cap);
+      total += (double)w * count;
+      n += parts * count;
+      item = std::max(item, (w + parts - 1) / parts);
+      if (parts > 1) shared += (double)parts / walks.size();
+    }
+    const double load = 1.7 * total / cus;
+    const double steps = equal ? std::max((double)((n + cus - 1) / cus) * item, load)
+                               : std::max((double)item, load + (walks.size() > 64 ? 1.0 : 0.5) * item);
+    return step_us * steps + (shared > 0 ? 8.0 + shared * elems * 8.0 / 4e6 : 0.0);
+  };
+  WalkShare best;
+  double t = expected(INT32_MAX);
+  for (int parts = 2; parts <= 16; ++parts) {
+    const int cap = (longest + parts - 1) / parts;
+    if (cap < 8 || parts * elems * 4.0 > 512e6) break;
+    const double x = expected(cap);
+    if (x < 0.9 * t) {
+      t = x;
+      best.cap = cap;
+      best.parts = (longest + cap - 1) / cap;
+    }
+  }
+  if (best.parts > 1 && walks.size() <= 64) {
+    auto share = [&](int w) { return best.cap >= w ? w : (w + (w + best.cap - 1) / best.cap - 1) / ((w + best.cap - 1) / best.cap); };
+    for (size_t i = 0; i < walks.size(); ++i) best.order[i] = (uint8_t)i;
+    std::stable_sort(best.order, best.order + walks.size(),
+                     [&](uint8_t x, uint8_t y) { return share(walks[x]) > share(walks[y]); });
+  }
+  return best;
+}
+
 // Attention backward: D-term pass, then dK/dV (one workgroup per 128 keys) and dQ (one per 256
 // queries), all reading the forward's lse; the D vector lives in the plan's workspace.
 int plan_attn_bwd(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
@@ -592,20 +644,62 @@ int plan_attn_bwd(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   a.q_bytes = (uint32_t)q_bytes;
   a.kv_bytes = (uint32_t)kv_bytes;
   a.D = d.D;
+  // Long walks over few blocks (grouped K/V heads: every query head of the group streams past each key
+  // block) are shared by several workgroups, whose partial sums a fourth kernel adds (B 2, H 32/8, 2048 x
+  // 2048 causal, D 128: 256 key blocks of 8 to 128 query tiles, one per CU). Walks of up to 32 query
+  // tiles or 15 key tiles stay whole: a share's own prologue and the sum would eat the gain.
+  WalkShare skv, sq;
+  if (!wide) {
+    const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
+    const long long diag = (long long)d.S_kv - d.S_q;
+    std::vector<int> wk((size_t)a.k_blocks), wq((size_t)a.q_blocks);
+    for (int i = 0; i < a.k_blocks; ++i) {
+      const long long t0 = d.causal ? std::max(0LL, 128LL * i - diag) / 64 : 0;
+      wk[(size_t)i] = (int)(std::max(0LL, (d.S_q + 63) / 64 - t0) * (d.H / d.H_kv));
+    }
+    for (int i = 0; i < a.q_blocks; ++i) {
+      const long long end = d.causal ? std::min<long long>(d.S_kv, 256LL * (i + 1) + diag) : d.S_kv;
+      wq[(size_t)(d.causal ? a.q_blocks - 1 - i : i)] = end > 0 ? (int)((end + 63) / 64) : 0;  // causal: rank 0 last
+    }
+    const double step = d.D <= 64 ? 1.4 : 2.0;
+    if (*std::max_element(wk.begin(), wk.end()) > 32)
+      skv = share_walks(wk, (long long)d.B * d.H_kv, !d.causal, step, (double)kv_bytes, cus);
+    if (*std::max_element(wq.begin(), wq.end()) > 15)
+      sq = share_walks(wq, (long long)d.B * d.H, !d.causal, step, (double)q_bytes / 2, cus);
+  }
+  memcpy(a.kv_order, skv.order, sizeof skv.order);
+  memcpy(a.q_order, sq.order, sizeof sq.order);
+  a.kv_cap = skv.cap;
+  a.kv_parts = skv.parts;
+  a.q_cap = sq.cap;
+  a.q_parts = sq.parts;
   Launch pre, kv, q;
   pre.name = std::string("mtk_attn_bwd_pre_") + dt;
   pre.grid = (unsigned)(((long long)d.B * d.S_q * d.H + 15) / 16);
-  kv.name = std::string(wide ? "mtk_attn_bwd256_dkdv_" : "mtk_attn_bwd_dkdv_") + (wide ? "" : lay) + dt + cz;
-  kv.grid = (unsigned)((long long)a.k_blocks * d.B * d.H_kv);  // per K/V head: sums over its query heads
-  q.name = std::string(wide ? "mtk_attn_bwd256_dq_" : "mtk_attn_bwd_dq_") + (wide ? "" : lay) + dt + cz;
-  q.grid = (unsigned)((long long)a.q_blocks * d.B * d.H);
+  kv.name = std::string(wide ? "mtk_attn_bwd256_dkdv_" : "mtk_attn_bwd_dkdv_") + (wide ? "" : lay) + dt + cz +
+            (skv.parts > 1 ? "_shared" : "");
+  kv.grid = (unsigned)((long long)a.k_blocks * d.B * d.H_kv * skv.parts);  // per K/V head: sums over its query heads
+  q.name = std::string(wide ? "mtk_attn_bwd256_dq_" : "mtk_attn_bwd_dq_") + (wide ? "" : lay) + dt + cz +
+           (sq.parts > 1 ? "_shared" : "");
+  q.grid = (unsigned)((long long)a.q_blocks * d.B * d.H * sq.parts);
   q.block = wide ? 256 : 512;
   for (Launch *l : {&pre, &kv, &q}) {
     set_args(*l, a);
     p->launches.push_back(*l);
   }
-  // workspace: the scaled D-term, then the base-2 lse, [B][H][S_q] fp32 each
-  p->workspace = 2 * (((size_t)d.B * d.H * d.S_q * sizeof(float) + 255) & ~(size_t)255);
+  if (skv.parts > 1 || sq.parts > 1) {
+    Launch sum;
+    sum.name = std::string("mtk_attn_bwd_sum_") + dt;
+    sum.grid = (unsigned)(((2 * kv_bytes + q_bytes) / 16 + 255) / 256);
+    set_args(sum, a);
+    p->launches.push_back(sum);
+  }
+  // workspace: the scaled D-term, then the base-2 lse, [B][H][S_q] fp32 each, then the partial sums of
+  // shared walks (dK and dV, dQ)
+  p->lt_at = ((size_t)d.B * d.H * d.S_q * sizeof(float) + 255) & ~(size_t)255;
+  p->part_kv_at = 2 * p->lt_at;
+  p->part_q_at = p->part_kv_at + (skv.parts > 1 ? (size_t)skv.parts * 4 * kv_bytes : 0);
+  p->workspace = p->part_q_at + (sq.parts > 1 ? (size_t)sq.parts * 2 * q_bytes : 0);
   double pairs = (double)d.S_q * d.S_kv;
   if (d.causal) {
     pairs = 0;
@@ -905,8 +999,8 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   //   sequences of at most half a workgroup per CU: B 1, H 8, 1023 x 1023, D 128: 23.5 -> 12.7; 2048 x
   //     2048: 41 -> 35, causal 42 -> 24; but B 4, H 12, 512 x 512, D 64 (192 blocks): 11.9 against 16.6.
   //     At D 128 one workgroup fits a CU: a second round of a few uncausal, short ones loses (B 3, H 16/4,
-  //     238 x 238, 360 workgroups: 10.5 against 14.4), as does D 64 (two per CU) below 512 keys (10 x 4
-  //     heads, 247 x 247: 8.0 against 9.3); causal ones are uneven anyway.
+  //     238 x 238, 360 workgroups: 10.5 against 14.4), as do D 64 (two per CU) and causal ones
+  //     (uneven anyway) below 512 keys (10 x 4 heads, 247 x 247, D 64: 8.0 against 9.3).
   //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the
   //     plan's choice (its kernel-select is fixed for such shapes; 4 x 1000 x 1000: 23 against 11).
   //   fewer than 4 key tiles leave too many wavefronts without one (28 x 8 heads, 3 x 34: 5.4 against 5.8);
@@ -917,7 +1011,7 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   const long long wgs = units * ((blocks32 + full - 1) / full);
   const bool full_rounds = wgs <= cus || d.H_kv < d.H || wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus);
   const bool decode = d.S_q <= 16 && key_tiles >= 8 ? full_rounds : d.S_q <= 64 && wgs <= cus;
-  const bool one_round = wgs <= cus || d.causal || (dp == 128 ? key_tiles >= 32 && wgs * 2 >= 3LL * cus : key_tiles >= 16);
+  const bool one_round = wgs <= cus || (dp == 128 && !d.causal ? key_tiles >= 32 && wgs * 2 >= 3LL * cus : key_tiles >= 16);
   const bool few = blocks * 2 <= cus && key_tiles >= 8 && one_round && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
   if (d.q_rows == 0 && !gen && !wide && key_tiles >= 4 && (decode || few)) {
     // fewer output blocks per workgroup while all workgroups still run at once: K is read again from
@@ -1125,7 +1219,9 @@ int bind_args(const mtk_plan *p, const void *argset, std::vector<Launch> &ls, vo
       a.dO = t->dO;
       a.lse = t->lse;
       a.Dt = (float *)t->workspace;
-      a.Lt = (float *)((char *)t->workspace + p->workspace / 2);
+      a.Lt = (float *)((char *)t->workspace + p->lt_at);
+      a.part_kv = (float *)((char *)t->workspace + p->part_kv_at);
+      a.part_q = (float *)((char *)t->workspace + p->part_q_at);
       a.dQ = t->dQ;
       a.dK = t->dK;
       a.dV = t->dV;
