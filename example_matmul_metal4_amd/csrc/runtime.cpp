@@ -558,12 +558,13 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
 // elems: fp32 values of one set of partial sums. One workgroup fits a CU; the shares are dispatched
 // longest first, so the last ends about half of the longest share after the average (more than 64
 // blocks, which are not sorted by share: a whole one; uncausal: equal walks, whole rounds). Partial
-// sums are written and read once, at about 4 TB/s.
+// sums are written and read once, at about 4 TB/s; sum_us: the sum's launch, where this adds it.
 struct WalkShare {
   int cap = INT32_MAX, parts = 1;
   uint8_t order[64] = {};  // indices into walks, longest share first
 };
-WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal, double step_us, double elems, int cus) {
+WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal, double step_us, double elems, double sum_us,
+                      int cus) {
   const int longest = *std::max_element(walks.begin(), walks.end());
   auto expected = [&](int cap) {
     double total = 0, shared = 0;
@@ -579,7 +580,7 @@ WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal
     const double load = 1.7 * total / cus;
     const double steps = equal ? std::max((double)((n + cus - 1) / cus) * item, load)
                                : std::max((double)item, load + (walks.size() > 64 ? 1.0 : 0.5) * item);
-    return step_us * steps + (shared > 0 ? 8.0 + shared * elems * 8.0 / 4e6 : 0.0);
+    return step_us * steps + (shared > 0 ? sum_us + shared * elems * 8.0 / 4e6 : 0.0);
   };
   WalkShare best;
   double t = expected(INT32_MAX);
@@ -663,9 +664,9 @@ int plan_attn_bwd(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
     }
     const double step = d.D <= 64 ? 1.4 : 2.0;
     if (*std::max_element(wk.begin(), wk.end()) > 32)
-      skv = share_walks(wk, (long long)d.B * d.H_kv, !d.causal, step, (double)kv_bytes, cus);
+      skv = share_walks(wk, (long long)d.B * d.H_kv, !d.causal, step, (double)kv_bytes, 8.0, cus);
     if (*std::max_element(wq.begin(), wq.end()) > 15)
-      sq = share_walks(wq, (long long)d.B * d.H, !d.causal, step, (double)q_bytes / 2, cus);
+      sq = share_walks(wq, (long long)d.B * d.H, !d.causal, step, (double)q_bytes / 2, skv.parts > 1 ? 0.0 : 8.0, cus);
   }
   memcpy(a.kv_order, skv.order, sizeof skv.order);
   memcpy(a.q_order, sq.order, sizeof sq.order);

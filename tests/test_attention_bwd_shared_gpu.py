@@ -14,7 +14,7 @@ CASES = [
     (1, 8, 1, 333, 300, 128, False, "f16", True, False), (1, 16, 2, 400, 417, 64, True, "bf16", True, False),
     (2, 12, 1, 257, 200, 72, True, "f16", True, False), (1, 2, 1, 1100, 1090, 128, True, "f16", True, True),
     (1, 1, 1, 300, 1500, 96, False, "bf16", False, True), (1, 1, 1, 1601, 1400, 64, True, "f16", False, True),
-    (1, 1, 1, 2200, 130, 128, False, "f16", True, False), (1, 6, 2, 1030, 1025, 40, False, "f16", True, False),
+    (1, 1, 1, 2200, 130, 128, False, "f16", True, False), (1, 6, 2, 1030, 1025, 40, False, "f16", True, True),
     (1, 4, 1, 1200, 640, 128, True, "f16", True, False),  # queries that see no key
 ]
 
