@@ -25,10 +25,11 @@
   }
 
 // the four 64x64 quarters of a 128x128 tile as workgroups, K-tiles over 8 wavefronts (two per SIMD)
-#define MTK_QUARTER_KERNEL(SUFFIX, AT, BN, ANY)                                                                 \
-  extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))                  \
+// (suffix q4: 4, two workgroups per CU)
+#define MTK_QUARTER_KERNEL(SUFFIX, AT, BN, ANY, W)                                                              \
+  extern "C" __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))               \
   MTK_GEMM_NAME(SUFFIX)(const mtk_tile_args a) {                                                               \
-    mtk::quarter_gemm<MTK_GEMM_DT, AT, BN, ANY, 8>(a);                                                          \
+    mtk::quarter_gemm<MTK_GEMM_DT, AT, BN, ANY, W>(a);                                                          \
   }
 
 namespace mtk_gemm_ops {
@@ -60,14 +61,22 @@ MTK_TILE_KERNEL(nt_128x128_v1, 128, 128, 2, 2, A_MK, B_NK, 1, 1)
 MTK_TILE_KERNEL(nn_256x256_v1, 256, 256, 2, 2, A_MK, B_KN, 1, 1)
 MTK_TILE_KERNEL(nn_128x128_v1, 128, 128, 2, 2, A_MK, B_KN, 1, 1)
 
-MTK_QUARTER_KERNEL(nt_128x128_dq, false, false, false)
-MTK_QUARTER_KERNEL(nn_128x128_dq, false, true, false)
-MTK_QUARTER_KERNEL(tt_128x128_dq, true, false, false)
-MTK_QUARTER_KERNEL(tn_128x128_dq, true, true, false)
-MTK_QUARTER_KERNEL(nt_128x128_v1q, false, false, true)
-MTK_QUARTER_KERNEL(nn_128x128_v1q, false, true, true)
-MTK_QUARTER_KERNEL(tt_128x128_v1q, true, false, true)
-MTK_QUARTER_KERNEL(tn_128x128_v1q, true, true, true)
+MTK_QUARTER_KERNEL(nt_128x128_dq, false, false, false, 8)
+MTK_QUARTER_KERNEL(nt_128x128_dq4, false, false, false, 4)
+MTK_QUARTER_KERNEL(nn_128x128_dq, false, true, false, 8)
+MTK_QUARTER_KERNEL(nn_128x128_dq4, false, true, false, 4)
+MTK_QUARTER_KERNEL(tt_128x128_dq, true, false, false, 8)
+MTK_QUARTER_KERNEL(tt_128x128_dq4, true, false, false, 4)
+MTK_QUARTER_KERNEL(tn_128x128_dq, true, true, false, 8)
+MTK_QUARTER_KERNEL(tn_128x128_dq4, true, true, false, 4)
+MTK_QUARTER_KERNEL(nt_128x128_v1q, false, false, true, 8)
+MTK_QUARTER_KERNEL(nt_128x128_v1q4, false, false, true, 4)
+MTK_QUARTER_KERNEL(nn_128x128_v1q, false, true, true, 8)
+MTK_QUARTER_KERNEL(nn_128x128_v1q4, false, true, true, 4)
+MTK_QUARTER_KERNEL(tt_128x128_v1q, true, false, true, 8)
+MTK_QUARTER_KERNEL(tt_128x128_v1q4, true, false, true, 4)
+MTK_QUARTER_KERNEL(tn_128x128_v1q, true, true, true, 8)
+MTK_QUARTER_KERNEL(tn_128x128_v1q4, true, true, true, 4)
 
 extern "C" __global__ void __launch_bounds__(256) MTK_REDUCE_NAME(const mtk_reduce_args a) {
   mtk::splitk_reduce<MTK_GEMM_DT>(a);

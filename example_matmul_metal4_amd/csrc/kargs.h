@@ -9,7 +9,7 @@
 
 #include <stdint.h>
 
-#define MTK_KARGS_VERSION 13
+#define MTK_KARGS_VERSION 14
 
 /* In-workgroup split-K: bytes of workspace slot per output tile of BM x BM (256 or 128). Each
  * wavefront keeps these accumulator blocks (32 x 32 fp32, 4 KB) of its running sum in the slot,
@@ -48,6 +48,10 @@ typedef struct {
   int32_t cDZ, cDY, cDX;
   int32_t cPF, cPT, cPL;
   int32_t cOD, cOH, cOW;
+  /* n / d for 0 <= n < 2^31 as umulhi(n, mul) >> shift (mul = 0: d = 1), quarter-tile convolutions */
+  struct {
+    uint32_t mul, shift;
+  } dOW, dOH, dOD, dC, dKW, dKH;
 } mtk_tile_args;
 
 /* Second pass of split-K: out[m][n] = sum_s partial[s][m][n] + bias[n]. */

@@ -32,7 +32,7 @@ struct QuarterOp {
     step_i = 16u * (uint32_t)ld;
     step_k = KMAJOR ? 128u * (uint32_t)ld : 128u;
   }
-  __device__ __forceinline__ void load(rsrc_t r, int kt, u32x4 (&v)[8], uint32_t (&e)[8]) const {
+  __device__ __forceinline__ void load(rsrc_t r, int kt, int, u32x4 (&v)[8], uint32_t (&e)[8]) const {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t off = lane_off + ((uint32_t)i * step_i + (uint32_t)kt * step_k);
@@ -78,8 +78,73 @@ struct QuarterOp {
   }
 };
 
-template <int DT, bool AT, bool BN, bool ANY, int W>
-__device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
+// The activation of an implicit-GEMM convolution as the row operand: row m is output pixel (n, oz, oh,
+// ow), K element ((kd * KH + kh) * KW + kw) * C + c. With C a multiple of 8 a chunk of 8 lies in one
+// filter tap: every lane decodes its chunk's tap once per K-tile and adds it to its 8 rows' window
+// origins; rows for which that tap lies in the padding (one bit per tap and dimension, up to 10 taps
+// each) and chunks past K are loaded out of range, as zeros.
+template <bool ANY>
+struct QuarterConv {
+  const mtk_tile_args &a;
+  int base[8];       // element offset of the row's window origin (may be negative)
+  uint32_t taps[8];  // in-range taps: depth | height << 10 | width << 20
+  uint32_t mis;
+
+  template <typename D>
+  static __device__ __forceinline__ int div(int n, const D &d) {
+    return d.mul ? (int)(__umulhi((uint32_t)n, d.mul) >> d.shift) : n;
+  }
+  __device__ void init(int lane, int first, int, uint32_t m) {
+    mis = m;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = first + 8 * i + (lane >> 3);
+      const int t1 = div(row, a.dOW), ow = row - t1 * a.cOW;
+      const int t2 = div(t1, a.dOH), oh = t1 - t2 * a.cOH;
+      const int n = div(t2, a.dOD), oz = t2 - n * a.cOD;
+      const int iz = oz * a.cSZ - a.cPF, ih = oh * a.cSY - a.cPT, iw = ow * a.cSX - a.cPL;
+      uint32_t t = 0;
+      for (int k = 0; k < a.cKD; ++k) t |= (uint32_t)((uint32_t)(iz + k * a.cDZ) < (uint32_t)a.cD) << k;
+      for (int k = 0; k < a.cKH; ++k) t |= (uint32_t)((uint32_t)(ih + k * a.cDY) < (uint32_t)a.cH) << (10 + k);
+      for (int k = 0; k < a.cKW; ++k) t |= (uint32_t)((uint32_t)(iw + k * a.cDX) < (uint32_t)a.cW) << (20 + k);
+      taps[i] = row < a.M ? t : 0;
+      base[i] = (((n * a.cD + iz) * a.cH + ih) * a.cW + iw) * a.cC;
+    }
+  }
+  __device__ __forceinline__ void load(rsrc_t r, int kt, int lane, u32x4 (&v)[8], uint32_t (&e)[8]) const {
+    const int k = kt * kBK + 8 * (lane & 7);
+    const int tap = div(k, a.dC), c = k - tap * a.cC;
+    const int t = div(tap, a.dKW), kw = tap - t * a.cKW;
+    const int kd = div(t, a.dKH), kh = t - kd * a.cKH;
+    const int at = ((kd * a.cDZ * a.cH + kh * a.cDY) * a.cW + kw * a.cDX) * a.cC + c;
+    const uint32_t need = k < a.K ? 1u << kd | 1u << (10 + kh) | 1u << (20 + kw) : ~0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t off = (taps[i] & need) == need ? (uint32_t)(base[i] + at) * 2u : kOOBAny;
+      v[i] = buf_load16(r, off);
+      if constexpr (ANY) e[i] = buf_load4(r, off + 16u);
+    }
+  }
+  __device__ __forceinline__ void store(char *lds, int lane, int, int, u32x4 (&v)[8], const uint32_t (&e)[8]) const {
+    const int r0 = lane >> 3, c = lane & 7;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      u32x4 w = v[i];
+      if constexpr (ANY) {  // chunks are 16 bytes apart: all as the activation itself starts
+        const uint32_t sh = mis << 3;
+        w = u32x4{__builtin_amdgcn_alignbit(w.y, w.x, sh), __builtin_amdgcn_alignbit(w.z, w.y, sh),
+                  __builtin_amdgcn_alignbit(w.w, w.z, sh), __builtin_amdgcn_alignbit(e[i], w.w, sh)};
+      }
+      *(u32x4 *)(lds + lds_off(8 * i + r0, c)) = w;
+    }
+  }
+  __device__ __forceinline__ u32x4 frag(const char *lds, int lane, int b, int ks) const {
+    return *(const u32x4 *)(lds + lds_off(32 * b + (lane & 31), 2 * ks + (lane >> 5)));
+  }
+};
+
+template <int DT, class AOp, bool BN, bool ANY, int W>
+__device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
   constexpr int kWaveB = 2 * 64 * 128;
   __shared__ __attribute__((aligned(1024))) char smem[W * kWaveB];
 
@@ -100,7 +165,6 @@ __device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
   uint32_t mis_a = 0, mis_b = 0;
   const rsrc_t ra = ANY ? make_rsrc_any(a.A, a.a_bytes, mis_a) : make_rsrc(a.A, a.a_bytes);
   const rsrc_t rb = ANY ? make_rsrc_any(a.B, a.b_bytes, mis_b) : make_rsrc(a.B, a.b_bytes);
-  QuarterOp<AT, ANY> oa;
   QuarterOp<BN, ANY> ob;
   oa.init(lane, m0, a.lda, mis_a);
   ob.init(lane, n0, a.ldb, mis_b);
@@ -111,15 +175,15 @@ __device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
   uint32_t ea[8], eb[8];
   int kt = kt0 + wave;
   if (kt < kt1) {
-    oa.load(ra, kt, sa, ea);
-    ob.load(rb, kt, sb, eb);
+    oa.load(ra, kt, lane, sa, ea);
+    ob.load(rb, kt, lane, sb, eb);
   }
   for (; kt < kt1; kt += W) {
     oa.store(la, lane, kt, a.K - kt * kBK, sa, ea);
     ob.store(lb, lane, kt, a.K - kt * kBK, sb, eb);
     if (kt + W < kt1) {
-      oa.load(ra, kt + W, sa, ea);
-      ob.load(rb, kt + W, sb, eb);
+      oa.load(ra, kt + W, lane, sa, ea);
+      ob.load(rb, kt + W, lane, sb, eb);
     }
     // this wavefront's own region: LDS accesses of a wavefront complete in order, the compiler has to
     // keep the reads of other lanes' chunks behind the writes
@@ -171,6 +235,17 @@ __device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
         if (row + r < a.M) C[(size_t)(row + r) * a.ldc] = to_bits<DT>(v[r] + bv);
     }
   }
+}
+
+template <int DT, bool AT, bool BN, bool ANY, int W>
+__device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
+  quarter_tile<DT, QuarterOp<AT, ANY>, BN, ANY, W>(a, QuarterOp<AT, ANY>{});
+}
+
+// Convolution: weights [K][O] as the K-major operand.
+template <int DT, bool ANY, int W>
+__device__ __forceinline__ void quarter_conv(const mtk_tile_args &a) {
+  quarter_tile<DT, QuarterConv<ANY>, true, ANY, W>(a, QuarterConv<ANY>{a});
 }
 
 }  // namespace mtk

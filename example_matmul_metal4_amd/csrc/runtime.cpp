@@ -216,36 +216,43 @@ float bf16_to_f32(uint16_t h) {
 
 // ------------------------------------------------------------------ GEMM planning
 
-// K partitions of a GEMM on quarter tiles (quarter.hpp: 64x64 workgroups whose 8 wavefronts share the
-// K-tiles), or 0 where the 128x128 tiles are expected to be faster. Chosen by expected time, in us,
-// from launches of 40 shapes on one box (kt: K-tiles of 64; about one workgroup of either kind per CU
-// and round at these sizes):
-//   quarter tiles   1.7 + rounds * (2.5 + 0.20 kt / split)        (rows of any alignment: 0.33)
-//   128x128 tiles   3.6 + 0.57 kt / split, up to 256 workgroups   (1.7)
+// A GEMM on quarter tiles (quarter.hpp: 64x64 workgroups whose wavefronts share the K-tiles): K
+// partitions and wavefronts per workgroup, or none where the 128x128 tiles are expected to be faster.
+// Chosen by expected time, in us, from launches of 70 shapes on one box (kt: K-tiles of 64):
+//   8 wavefronts, one workgroup per CU    1.7 + rounds * (2.5 + 0.20 kt / split)    (any alignment: 0.33)
+//   4 wavefronts, two workgroups per CU   1.7 + half rounds * (3.6 + 0.41 kt)       (0.62)
+//   128x128 tiles                         3.6 + 0.57 kt / split, up to 256          (1.7)
 //   two or more partitions add a second kernel and its partial sums: 3.5 (quarters), 4.5
-// Measured, 128x128 -> quarters, no split: 1024 cubed 13.3 -> 7.5; 1024 x 1024 x 4096 39.0 -> 17.4; 512 x
-// 512 x 1024 10.0 -> 6.9; 256 cubed 5.7 -> 4.9; 1024 x 2048 x 2048 22.4 -> 19.1; but 640 x 3072 x 768 11.9
-// against 12.4, 1536 cubed 18.6 against 27.0. The plan's own split: 256 x 4096 x 4096 20.4 -> 16.6, 64 x
-// 4096 x 14336 36.7 -> 28.6, but 310 x 2160 x 6864 24.6 against 33.4. Odd leading dimensions, no split:
-// 1023 cubed 31.0 -> 10.5, 2047 x 2047 x 4095 112 -> 94.
-int quarter_split(int M, int N, int k_tiles, int split_k, bool direct, int cus) {
-  if (k_tiles < 4) return 0;  // nothing to share out
+// Measured, 128x128 -> quarters, no split: 1024 cubed 13.3 -> 7.6; 1024 x 1024 x 4096 39.0 -> 17.4; 512 x
+// 512 x 1024 10.0 -> 6.9; 256 cubed 5.7 -> 4.9; 1024 x 2048 x 2048 22.4 -> 18.5 (4 wavefronts; 8: 20.6); 640 x
+// 3072 x 768 11.9 -> 10.9; but 2048 x 1024 x 256 6.5 against 7.0, 1536 cubed 18.6 against 22.4. The plan's
+// own split: 256 x 4096 x 4096 20.4 -> 16.6, 64 x 4096 x 14336 36.7 -> 28.6, but 310 x 2160 x 6864 24.6 against
+// 33.4. Odd leading dimensions, no split: 1023 cubed 31.0 -> 10.2, 2047 x 2047 x 4095 112 -> 87.
+struct Quarter {
+  int split = 0, waves = 8;
+};
+Quarter quarter_plan(int M, int N, int k_tiles, int split_k, bool direct, int cus) {
+  Quarter best;
+  if (k_tiles < 4) return best;  // nothing to share out
   const long long q = (long long)((M + 63) / 64) * ((N + 63) / 64);
   const long long t = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  const double kq = direct ? 0.20 : 0.33, k128 = direct ? 0.57 : 1.7;
-  if (t > cus) return 0;
-  auto quarters = [&](int s) {
-    const double rounds = (double)((q * s + cus - 1) / cus);
-    return 1.7 + rounds * (2.5 + kq * ((k_tiles + s - 1) / s)) + (s > 1 ? 3.5 : 0.0);
-  };
+  if (t > cus) return best;
   int s128 = 1;  // the split that 128x128 tiles would take
   if (split_k == 0 && t * 4 < 3LL * cus) s128 = (int)std::min<long long>({cus / t, std::max(1, k_tiles / 4), 16LL});
-  const double tiles = 3.6 + k128 * ((k_tiles + s128 - 1) / s128) + (s128 > 1 ? 4.5 : 0.0);
-  int best = 1;
-  if (split_k == 0)
-    for (int s = 2; s <= 16 && q * s <= cus && k_tiles >= 6 * s; ++s)
-      if (quarters(s) < quarters(best)) best = s;
-  return quarters(best) < tiles ? best : 0;
+  double expected = 3.6 + (direct ? 0.57 : 1.7) * ((k_tiles + s128 - 1) / s128) + (s128 > 1 ? 4.5 : 0.0);
+  auto consider = [&](int split, int waves, double us) {
+    if (us >= expected) return;
+    expected = us;
+    best.split = split;
+    best.waves = waves;
+  };
+  for (int s = 1; s == 1 || (split_k == 0 && s <= 16 && q * s <= cus && k_tiles >= 6 * s); ++s) {
+    const double rounds = (double)((q * s + cus - 1) / cus);
+    consider(s, 8, 1.7 + rounds * (2.5 + (direct ? 0.20 : 0.33) * ((k_tiles + s - 1) / s)) + (s > 1 ? 3.5 : 0.0));
+  }
+  const double rounds = std::max(1.0, 0.5 * (double)((q + cus - 1) / cus));
+  if (q > cus) consider(1, 4, 1.7 + rounds * (3.6 + (direct ? 0.41 : 0.62) * k_tiles));
+  return best;
 }
 
 int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
@@ -425,13 +432,13 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   int split = d.split_k;
   // Quarter tiles: only where neither a tile, a partition layout nor a schedule is asked for; and for A
   // [K][M] with odd rows of B always (no other kernel reads them).
-  int quarter = 0;
+  Quarter quarter;
   if (tile == 0 && d.split_mode == MTK_SPLIT_AUTO && d.k_stagger == 0 && split <= 1)
-    quarter = quarter_split(d.M, d.N, k_tiles, split, direct, ctx ? ctx->prop.multiProcessorCount : 256);
-  if (d.trans_a && !direct && !quarter && d.split_mode != MTK_SPLIT_SERIAL) quarter = std::max(1, split);
-  if (quarter) {
+    quarter = quarter_plan(d.M, d.N, k_tiles, split, direct, ctx ? ctx->prop.multiProcessorCount : 256);
+  if (d.trans_a && !direct && !quarter.split && d.split_mode != MTK_SPLIT_SERIAL) quarter = {std::max(1, split), 4};
+  if (quarter.split) {
     tile = 128;
-    split = quarter;
+    split = quarter.split;
   }
   if (tile == 0) {
     // 256x256 tiles when there are enough of them (with the requested split) to fill most of the
@@ -445,7 +452,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     // other's loads (4095 cubed, f16: 252 us against 566 us on 256x256, one wavefront per SIMD)
     if (d.lda % 2 != 0 || d.ldb % 2 != 0) tile = 128;
   }
-  const int edge = quarter ? 64 : tile;  // of a workgroup's tile
+  const int edge = quarter.split ? 64 : tile;  // of a workgroup's tile
   const int tiles_m = (d.M + edge - 1) / edge, tiles_n = (d.N + edge - 1) / edge;
   const long long tiles = (long long)tiles_m * tiles_n;
   if (split == 0) {  // fill about one wave of 256 CUs with split-K when the tile grid is small
@@ -462,7 +469,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   // fills the device (every CU busy without extra partition workgroups), and it saves the second
   // kernel and 1/split of the partial traffic.
   bool serial = false;
-  if (split > 1 && !quarter) {
+  if (split > 1 && !quarter.split) {
     const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
     if (d.split_mode == MTK_SPLIT_SERIAL) {
       if (split > 4 || !direct) {
@@ -480,9 +487,9 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   char name[96];
   // operand letters: A [M][K] 'n' / [K][M] 't', B [N][K] 't' / [K][N] 'n'
   snprintf(name, sizeof name, "mtk_gemm_%s_%c%c_%dx%d_%s%s", dt, d.trans_a ? 't' : 'n', d.trans_b ? 't' : 'n', tile,
-           tile, serial ? "s" : direct ? "d" : "v1", quarter ? "q" : "");
+           tile, serial ? "s" : direct ? "d" : "v1", !quarter.split ? "" : quarter.waves == 4 ? "q4" : "q");
   g.name = name;
-  if (quarter) g.block = 512;
+  if (quarter.split) g.block = 64u * (unsigned)quarter.waves;
   if (tile == 256 && direct) g.block = 512;  // 256x256 direct-to-LDS tiles run 8 wavefronts
   g.grid = (unsigned)(serial ? tiles : tiles * split);
   mtk_tile_args a{};
@@ -540,7 +547,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
            "gemm %s %s %s M=%d N=%d K=%d tile=%dx%d split_k=%d k_tiles/split=%d k_stagger=%d %s grid=%u%s", dt,
            d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, tile, tile, split, kps,
            a.k_stagger,
-           quarter ? "64x64 quarters, K-tiles over 8 wavefronts" : direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
+           quarter.split ? "64x64 quarters, K-tiles over the wavefronts" : direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
            serial ? " (partitions in sequence per tile, summed in the epilogue)" : split > 1 ? " + splitk_reduce" : "");
   p->description = desc;
   int s = resolve(p);
@@ -808,6 +815,38 @@ int normalise_conv(const mtk_conv_desc *in, mtk_conv_desc *d) {
   return MTK_OK;
 }
 
+// Multiplier and shift of kargs.h's division by d: m = ceil(2^(31 + l) / d) with 2^l >= d > 2^(l - 1) fits
+// 32 bits, and n * (m d - 2^(31 + l)) / d < 2^(31 + l) / d for n < 2^31, so the quotient is exact.
+template <typename D>
+void set_divisor(D &out, int d) {
+  out.mul = out.shift = 0;
+  if (d <= 1) return;
+  int l = 1;
+  while ((1ll << l) < d) ++l;
+  out.mul = (uint32_t)(((1ull << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d);
+  out.shift = (uint32_t)(l - 1);
+}
+
+// Wavefronts per workgroup of a convolution on quarter tiles (quarter.hpp; channels in multiples of 8,
+// up to 10 taps per dimension), or 0 for the 128x128 / 256x256 tiles. One box, us:
+//   at most one 64x64 quarter per CU: 8 wavefronts. 702 pixels x 64, 256 channels 3x3: 25.9 -> 13.6; 16384 x
+//     32, 32 channels 3x3: 11.9 -> 8.0; 7488 x 128, 512 channels 3x3x3: 137 -> 49
+//   at most two: 4 wavefronts, two workgroups per CU. 3186 x 512, 512 channels 3x3: 51.7 -> 35.1 (8: 40.3)
+//   more, where 128 columns are half empty (up to 64 output channels) and the walk is long: 658812 x 32, 64
+//     channels 3x3x3: 312 -> 279; 57138 x 32, 256 channels 3x3: 43.2 -> 42.5; with channels that are not a multiple
+//     of 64 (the 128x128 kernel decodes a tap per chunk) shorter ones too: 311808 x 16, 32 channels 3x3x3: 124
+//     -> 100; and up to three rounds of any width: 22960 x 72, 96 channels 5x5: 64.8 -> 38.6
+//   otherwise the 128x128 tiles: 28749 x 512, 96 channels 3x3: 56.6 against 79.9
+//   one or two K-tiles: nothing to share (20400 x 256, 32 channels 1x1: 9.8 against 18.2)
+int conv_quarter(long long M, const mtk_conv_desc &d, int k_tiles, bool fast, int cus) {
+  if (d.C % 8 != 0 || d.KD > 10 || d.KH > 10 || d.KW > 10 || k_tiles < 3 || M >= (1 << 30)) return 0;
+  const long long q = (M + 63) / 64 * ((d.O + 63) / 64);
+  if (q <= cus) return 8;
+  if (q <= 2LL * cus) return 4;
+  if (d.O <= 64 && k_tiles >= (fast ? 20 : 7)) return 4;
+  return !fast && q <= 3LL * cus && k_tiles >= 12 ? 4 : 0;
+}
+
 int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
   if (!out) return fail(MTK_ERR_INVALID, "null output");
   mtk_conv_desc d;
@@ -919,6 +958,19 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
   a.cOD = od;
   a.cOH = oh;
   a.cOW = ow;
+  const int quarter = conv_quarter(M, d, a.k_tiles, fast, ctx ? ctx->prop.multiProcessorCount : 256);
+  if (quarter) {
+    g.name = std::string("mtk_conv_f16_gen_128x128_") + (!fast && va == 1 ? "v1q" : "q") + std::to_string(quarter);
+    g.block = 64 * quarter;
+    a.tiles_m = (int)((M + 63) / 64);
+    a.tiles_n = (d.O + 63) / 64;
+    set_divisor(a.dOW, ow);
+    set_divisor(a.dOH, oh);
+    set_divisor(a.dOD, od);
+    set_divisor(a.dC, d.C);
+    set_divisor(a.dKW, d.KW);
+    set_divisor(a.dKH, d.KH);
+  }
   g.grid = (unsigned)((long long)a.tiles_m * a.tiles_n);
   set_args(g, a);
   p->launches.push_back(g);
@@ -927,7 +979,7 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
              (oidhw ? 2.0 * (double)w_bytes : 0.0);  // the re-layout reads and writes the weights once
   char desc[288];
   snprintf(desc, sizeof desc, "conv%dd f16 implicit-GEMM M=%lld N=%d K=%lld out=%dx%dx%d tile=%dx%d gather=%s grid=%u%s",
-           d.rank, M, d.O, K, od, oh, ow, bm, bn, kind, g.grid,
+           d.rank, M, d.O, K, od, oh, ow, quarter ? 64 : bm, quarter ? 64 : bn, kind, g.grid,
            oidhw ? " weights OIDHW (re-laid out in the workspace)" : "");
   p->description = desc;
   s = resolve(p);

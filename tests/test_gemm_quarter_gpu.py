@@ -1,5 +1,5 @@
-"""GEMMs on quarter tiles (64x64 workgroups whose wavefronts share the K-tiles): every operand layout,
-edges of the 64x64 tile, K-tiles that do and do not divide over the 8 wavefronts, K tails, padded and
+"""GEMMs on quarter tiles (64x64 workgroups whose 8 or 4 wavefronts share the K-tiles): every operand layout,
+edges of the 64x64 tile, K-tiles that do and do not divide over the wavefronts, K tails, padded and
 odd rows (NaN in the padding), and the plan's own K partitions. Against the CPU oracle."""
 import numpy as np
 import pytest
@@ -15,8 +15,11 @@ CASES = [(m, n, k, ta, tb, pa, pb, 1, dt)
          for (m, n, k, pa, pb, dt) in ((64, 64, 256, 0, 0, "f16"), (66, 63, 193, 0, 1, "bf16"), (2, 130, 700, 2, 4, "f16"),
                                        (190, 1, 577, 4, 1, "f16"), (1000, 900, 330, 0, 0, "bf16"))]
 CASES += [(60, 128, 9000, False, True, 0, 0, 0, "f16"), (130, 514, 2801, True, False, 0, 0, 0, "bf16"),
-          (9, 1001, 5003, False, True, 0, 0, 0, "f16"), (40, 70, 4097, False, False, 1, 1, 0, "f16"),
-          (4, 40, 70, True, True, 0, 1, 1, "f16"), (500, 100, 1025, True, True, 0, 0, 3, "f16")]
+          (9, 1001, 5003, False, True, 0, 0, 0, "f16"), (40, 70, 4097, False, False, 1, 1, 0, "f16")]
+# more than one quarter per CU, or a layout that no other kernel reads: 4 wavefronts per workgroup
+FOUR = [(4, 40, 70, True, True, 0, 1, 1, "f16"), (500, 100, 1025, True, True, 0, 0, 3, "f16"), (1100, 1030, 1300, False, True, 0, 0, 1, "f16"),
+        (1030, 1101, 517, False, False, 1, 0, 0, "bf16"), (1100, 1034, 1290, True, False, 0, 0, 1, "bf16")]
+CASES += FOUR
 
 
 def _plan(dev, case):
@@ -29,7 +32,7 @@ def test_which_plans_are_quartered():
     # CPU: the planner alone
     for c in CASES:
         kern = _plan(None, c).describe().split("kernels: ")[1].split()[0]
-        assert kern.endswith("q"), (c, kern)
+        assert kern.endswith("q4" if c in FOUR else "q"), (c, kern)
     assert "splitk_reduce" in _plan(None, CASES[20]).describe() and "splitk_reduce" in _plan(None, CASES[22]).describe()
     # larger grids, requested tiles, partitions or schedules, and K of fewer than four K-tiles are not
     for kw in (dict(M=2048, N=2048, K=512), dict(M=1024, N=1024, K=1024, tile=128), dict(M=512, N=512, K=4096, split_k=4),
