@@ -31,6 +31,12 @@
   MTK_GEMM_NAME(SUFFIX)(const mtk_tile_args a) {                                                               \
     mtk::quarter_gemm<MTK_GEMM_DT, AT, BN, ANY, W>(a);                                                          \
   }
+// the same with up to ROWS rows of A [M][K] per workgroup (suffix q<ROWS>)
+#define MTK_QUARTER_TALL_KERNEL(SUFFIX, BN, ROWS, W)                                                            \
+  extern "C" __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))               \
+  MTK_GEMM_NAME(SUFFIX)(const mtk_tile_args a) {                                                               \
+    mtk::quarter_tall<MTK_GEMM_DT, BN, ROWS, W>(a);                                                             \
+  }
 
 namespace mtk_gemm_ops {
 using R256 = mtk::OpRows<256, 8>;
@@ -77,6 +83,8 @@ MTK_QUARTER_KERNEL(tt_128x128_v1q, true, false, true, 8)
 MTK_QUARTER_KERNEL(tt_128x128_v1q4, true, false, true, 4)
 MTK_QUARTER_KERNEL(tn_128x128_v1q, true, true, true, 8)
 MTK_QUARTER_KERNEL(tn_128x128_v1q4, true, true, true, 4)
+MTK_QUARTER_TALL_KERNEL(nt_128x128_dq96, false, 96, 8)
+MTK_QUARTER_TALL_KERNEL(nn_128x128_dq96, true, 96, 8)
 
 extern "C" __global__ void __launch_bounds__(256) MTK_REDUCE_NAME(const mtk_reduce_args a) {
   mtk::splitk_reduce<MTK_GEMM_DT>(a);

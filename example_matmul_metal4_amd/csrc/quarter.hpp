@@ -3,7 +3,7 @@
 //
 // With one 128x128 tile per CU or fewer, a K loop that all wavefronts walk together costs one memory
 // latency per K-tile (about 1.5 us: 1023 cubed has 64 tiles of 16 K-tiles, 31 us for 2.1 GFLOP). Here
-//   * every wavefront takes every W-th K-tile of 64 for the whole 64x64 quarter (2 x 2 blocks of
+//   * every wavefront takes every W-th K-tile of 64 for the whole 64x64 quarter (or 96x64 tile; 2 x 2 blocks of
 //     32x32x16 MFMAs: one fragment read per MFMA), staged global -> registers -> its own 16 KB of LDS:
 //     no barrier until the end, and the loads of its next tile in flight meanwhile (two tiles ahead
 //     was slower: registers, 18.4 -> 19.5 us at 1024 x 1024 x 4096);
@@ -16,9 +16,11 @@
 
 namespace mtk {
 
-// One operand of a 64x64x64 step: 64 rows of 64 K (KMAJOR false) or 64 K rows of 64 columns.
-template <bool KMAJOR, bool ANY>
+// One operand of a step of 64 K: ROWS rows of 64 K (KMAJOR false) or 64 K rows of 64 columns.
+template <bool KMAJOR, bool ANY, int ROWS = 64>
 struct QuarterOp {
+  static_assert(!KMAJOR || ROWS == 64, "K-major operands are 64 columns wide");
+  static constexpr int kRows = ROWS, kLoads = ROWS / 8;
   uint32_t lane_off;  // bytes: this lane's chunk of the first load instruction at K-tile 0
   uint32_t step_i;    // bytes between load instructions (8 rows)
   uint32_t step_k;    // bytes between K-tiles
@@ -32,9 +34,9 @@ struct QuarterOp {
     step_i = 16u * (uint32_t)ld;
     step_k = KMAJOR ? 128u * (uint32_t)ld : 128u;
   }
-  __device__ __forceinline__ void load(rsrc_t r, int kt, int, u32x4 (&v)[8], uint32_t (&e)[8]) const {
+  __device__ __forceinline__ void load(rsrc_t r, int kt, int, u32x4 (&v)[kLoads], uint32_t (&e)[kLoads]) const {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
       const uint32_t off = lane_off + ((uint32_t)i * step_i + (uint32_t)kt * step_k);
       if constexpr (ANY) {
         v[i] = buf_load16(r, off & ~3u);
@@ -45,10 +47,11 @@ struct QuarterOp {
     }
   }
   // The staged chunks to LDS; k: K elements from this K-tile on (< 64: the last, partial one).
-  __device__ __forceinline__ void store(char *lds, int lane, int kt, int k, u32x4 (&v)[8], const uint32_t (&e)[8]) const {
+  __device__ __forceinline__ void store(char *lds, int lane, int kt, int k, u32x4 (&v)[kLoads],
+                                        const uint32_t (&e)[kLoads]) const {
     const int r0 = lane >> 3, c = lane & 7;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < kLoads; ++i) {
       u32x4 w = v[i];
       if constexpr (ANY) {
         const uint32_t sh = ((lane_off + ((uint32_t)i * step_i + (uint32_t)kt * step_k)) & 2u) << 3;
@@ -73,7 +76,7 @@ struct QuarterOp {
       const u32x2 v = __builtin_bit_cast(u32x2, x), w = __builtin_bit_cast(u32x2, y);
       return u32x4{v.x, v.y, w.x, w.y};
     } else {
-      return *(const u32x4 *)(lds + lds_off(32 * b + (lane & 31), 2 * ks + (lane >> 5)));
+      return *(const u32x4 *)(lds + frag_off(32 * b, ks, lane));
     }
   }
 };
@@ -85,6 +88,7 @@ struct QuarterOp {
 // each) and chunks past K are loaded out of range, as zeros.
 template <bool ANY>
 struct QuarterConv {
+  static constexpr int kRows = 64, kLoads = 8;
   const mtk_tile_args &a;
   int base[8];       // element offset of the row's window origin (may be negative)
   uint32_t taps[8];  // in-range taps: depth | height << 10 | width << 20
@@ -139,13 +143,15 @@ struct QuarterConv {
     }
   }
   __device__ __forceinline__ u32x4 frag(const char *lds, int lane, int b, int ks) const {
-    return *(const u32x4 *)(lds + lds_off(32 * b + (lane & 31), 2 * ks + (lane >> 5)));
+    return *(const u32x4 *)(lds + frag_off(32 * b, ks, lane));
   }
 };
 
 template <int DT, class AOp, bool BN, bool ANY, int W>
 __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
-  constexpr int kWaveB = 2 * 64 * 128;
+  constexpr int MB = AOp::kRows / 32;                   // 32-row blocks
+  constexpr int kWaveB = (AOp::kRows + 64) * 128;
+  constexpr int kPasses = MB * 8192 <= kWaveB ? 1 : 2;  // of the final sum: both column blocks at once, or one each
   __shared__ __attribute__((aligned(1024))) char smem[W * kWaveB];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -158,7 +164,7 @@ __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
   const int group = kGroupM * a.tiles_n;
   const int first_m = (t / group) * kGroupM;
   const int gm = min(a.tiles_m - first_m, kGroupM);
-  const int m0 = (first_m + (t % group) % gm) * 64, n0 = (t % group) / gm * 64;
+  const int m0 = (first_m + (t % group) % gm) * AOp::kRows, n0 = (t % group) / gm * 64;
   const int kt0 = split_first_tile(a, split, t);
   const int kt1 = split_first_tile(a, split + 1, t);
 
@@ -168,11 +174,11 @@ __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
   QuarterOp<BN, ANY> ob;
   oa.init(lane, m0, a.lda, mis_a);
   ob.init(lane, n0, a.ldb, mis_b);
-  char *la = smem + wave * kWaveB, *lb = la + 64 * 128;
+  char *la = smem + wave * kWaveB, *lb = la + AOp::kRows * 128;
 
-  f32x16 acc[2][2] = {};
-  u32x4 sa[8], sb[8];
-  uint32_t ea[8], eb[8];
+  f32x16 acc[MB][2] = {};
+  u32x4 sa[AOp::kLoads], sb[8];
+  uint32_t ea[AOp::kLoads], eb[8];
   int kt = kt0 + wave;
   if (kt < kt1) {
     oa.load(ra, kt, lane, sa, ea);
@@ -191,10 +197,12 @@ __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int ks = 0; ks < kBK / 16; ++ks) {
-      const u32x4 fa[2] = {oa.frag(la, lane, 0, ks), oa.frag(la, lane, 1, ks)};
+      u32x4 fa[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[i] = oa.frag(la, lane, i, ks);
       const u32x4 fb[2] = {ob.frag(lb, lane, 0, ks), ob.frag(lb, lane, 1, ks)};
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x16<DT>(fa[i], fb[j], acc[i][j]);
     }
@@ -203,36 +211,42 @@ __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
   }
 
   // ---- add the wavefronts' sums: accumulator quads parked as [block][quad][lane], 16 bytes each
-  f32x4 *park = (f32x4 *)(smem + wave * kWaveB);  // own region
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const f32x16 &x = acc[b >> 1][b & 1];
-      park[(4 * b + q) * 64 + lane] = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
-    }
-  __syncthreads();
+  constexpr int kCols = 2 / kPasses;  // column blocks per pass
   const uint16_t *bias = (const uint16_t *)a.bias;
 #pragma unroll
-  for (int it = tid; it < 1024; it += 64 * W) {
-    f32x4 s = *(const f32x4 *)(smem + it * 16);
+  for (int pass = 0; pass < kPasses; ++pass) {
+    if (pass > 0) __syncthreads();  // the pass before has been read
+    f32x4 *park = (f32x4 *)(smem + wave * kWaveB);  // own region
 #pragma unroll
-    for (int w = 1; w < W; ++w) s += *(const f32x4 *)(smem + w * kWaveB + it * 16);
-    const int b = it >> 8, q = (it >> 6) & 3, l = it & 63;
-    const int row = m0 + 32 * (b >> 1) + 8 * q + 4 * (l >> 5), col = n0 + 32 * (b & 1) + (l & 31);
-    if (col >= a.N) continue;
-    const float v[4] = {s.x, s.y, s.z, s.w};
-    if (a.partial != nullptr) {
-      float *P = a.partial + (size_t)split * a.M * a.N + col;
+    for (int b = 0; b < MB * kCols; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (row + r < a.M) P[(size_t)(row + r) * a.N] = v[r];
-    } else {
-      const float bv = a.has_bias ? from_bits<DT>(bias[col]) : 0.0f;
-      uint16_t *C = (uint16_t *)a.C + col;
+      for (int q = 0; q < 4; ++q) {
+        const f32x16 &x = acc[b / kCols][pass + b % kCols];
+        park[(4 * b + q) * 64 + lane] = f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+      }
+    __syncthreads();
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (row + r < a.M) C[(size_t)(row + r) * a.ldc] = to_bits<DT>(v[r] + bv);
+    for (int it = tid; it < MB * kCols * 256; it += 64 * W) {
+      f32x4 s = *(const f32x4 *)(smem + it * 16);
+#pragma unroll
+      for (int w = 1; w < W; ++w) s += *(const f32x4 *)(smem + w * kWaveB + it * 16);
+      const int b = it >> 8, q = (it >> 6) & 3, l = it & 63;
+      const int row = m0 + 32 * (b / kCols) + 8 * q + 4 * (l >> 5);
+      const int col = n0 + 32 * (pass + b % kCols) + (l & 31);
+      if (col >= a.N) continue;
+      const float v[4] = {s.x, s.y, s.z, s.w};
+      if (a.partial != nullptr) {
+        float *P = a.partial + (size_t)split * a.M * a.N + col;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (row + r < a.M) P[(size_t)(row + r) * a.N] = v[r];
+      } else {
+        const float bv = a.has_bias ? from_bits<DT>(bias[col]) : 0.0f;
+        uint16_t *C = (uint16_t *)a.C + col;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (row + r < a.M) C[(size_t)(row + r) * a.ldc] = to_bits<DT>(v[r] + bv);
+      }
     }
   }
 }
@@ -240,6 +254,16 @@ __device__ __forceinline__ void quarter_tile(const mtk_tile_args &a, AOp oa) {
 template <int DT, bool AT, bool BN, bool ANY, int W>
 __device__ __forceinline__ void quarter_gemm(const mtk_tile_args &a) {
   quarter_tile<DT, QuarterOp<AT, ANY>, BN, ANY, W>(a, QuarterOp<AT, ANY>{});
+}
+
+// 96 rows of A [M][K] per workgroup, for M where one or two such tiles replace two or three of 64 (B is read
+// once for more rows). HBM and the L2 reads of A bound it: 20 KB per K-tile and CU, 8 in flight (160 KB of
+// LDS, 254 VGPRs; a spill in the loop waits for the loads in flight: 41 us instead of 33). 77 x 4096 x 14336,
+// bf16: 38.0 us on 128x128 tiles, 39.6 on 64x64 quarters -> 33.0.
+template <int DT, bool BN, int ROWS, int W>
+__device__ __forceinline__ void quarter_tall(const mtk_tile_args &a) {
+  using A = QuarterOp<false, false, ROWS>;
+  quarter_tile<DT, A, BN, false, W>(a, A{});
 }
 
 // Convolution: weights [K][O] as the K-major operand.

@@ -229,7 +229,7 @@ float bf16_to_f32(uint16_t h) {
 // own split: 256 x 4096 x 4096 20.4 -> 16.6, 64 x 4096 x 14336 36.7 -> 28.6, but 310 x 2160 x 6864 24.6 against
 // 33.4. Odd leading dimensions, no split: 1023 cubed 31.0 -> 10.2, 2047 x 2047 x 4095 112 -> 87.
 struct Quarter {
-  int split = 0, waves = 8;
+  int split = 0, waves = 8, rows = 64;  // rows of a workgroup's tile
 };
 Quarter quarter_plan(int M, int N, int k_tiles, int split_k, bool direct, int cus) {
   Quarter best;
@@ -253,6 +253,34 @@ Quarter quarter_plan(int M, int N, int k_tiles, int split_k, bool direct, int cu
   const double rounds = std::max(1.0, 0.5 * (double)((q + cus - 1) / cus));
   if (q > cus) consider(1, 4, 1.7 + rounds * (3.6 + (direct ? 0.41 : 0.62) * k_tiles));
   return best;
+}
+
+// One or two 96-row tiles of A [M][K] (64 < M <= 96, 128 < M <= 192; even rows), 8 wavefronts: B is
+// read for all (or half the) rows at once, at 3.3 to 3.9 TB/s, where the tiles below reach 2.8 to 3.1. Taken
+// where B's columns (and enough K to share out) keep the CUs busy for long enough.
+// us, better of the others -> this, bf16 (partitions):
+//   77 x 4096 x 14336 (4) 37.8 -> 33.0, 77 x 14336 x 4096 (1) 40.9 -> 32.8, 90 x 16384 x 1024 (1) 14.4 -> 13.7, 66 x 5120 x 5120
+//   (3) 23.5 -> 21.4, 130 x 8192 x 8192 (1) 65.4 -> 46.0, 160 x 4096 x 14336 (2) 57.3 -> 47.5; but 66 x 8192 x 2048 (2) 14.0
+//   against 16.4, 77 x 1024 x 8192 (16) 11.1 against 13.0, 160 x 4096 x 4096 (2) 20.4 against 21.7; more workgroups than
+//   CUs, 93 x 29184 x 992, B [K][N]: 21.1 against 27.4
+// Over the 3589 of 5967 random shapes timed on both that it takes: geometric mean 1.19x, worst 0.90x, 3
+// below 0.97x; those it leaves (fewer busy CUs, two rounds): 1.05x, down to 0.77x.
+// Three 96-row tiles, and 128 rows for M up to 128 (whose registers spill), were slower than 128x128.
+Quarter tall_plan(int M, int N, int k_tiles, int split_k, bool b_rows, int cus) {
+  Quarter q;
+  const int tm = M > 64 && M <= 96 ? 1 : M > 128 && M <= 192 ? 2 : 0;
+  const long long wgs = tm * (long long)((N + 63) / 64);
+  if (!tm || wgs > cus) return q;
+  const int s = split_k == 1 ? 1 : (int)(cus / wgs);
+  const int steps = k_tiles / s;  // per partition
+  const long long busy = 100 * wgs * s / cus;  // percent of the CUs
+  const bool ok = s == 1 ? busy >= (tm == 1 ? 67 : 72) && steps >= 16
+                         : s <= 10 && busy >= (b_rows ? 86 : 95) && steps >= (tm == 2 ? 48 : s == 2 ? 40 : 16);
+  if (ok) {
+    q.split = s;
+    q.rows = 96;
+  }
+  return q;
 }
 
 int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
@@ -433,8 +461,11 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   // Quarter tiles: only where neither a tile, a partition layout nor a schedule is asked for; and for A
   // [K][M] with odd rows of B always (no other kernel reads them).
   Quarter quarter;
-  if (tile == 0 && d.split_mode == MTK_SPLIT_AUTO && d.k_stagger == 0 && split <= 1)
-    quarter = quarter_plan(d.M, d.N, k_tiles, split, direct, ctx ? ctx->prop.multiProcessorCount : 256);
+  if (tile == 0 && d.split_mode == MTK_SPLIT_AUTO && d.k_stagger == 0 && split <= 1) {
+    const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
+    if (direct && !d.trans_a) quarter = tall_plan(d.M, d.N, k_tiles, split, d.trans_b, cus);
+    if (!quarter.split) quarter = quarter_plan(d.M, d.N, k_tiles, split, direct, cus);
+  }
   if (d.trans_a && !direct && !quarter.split && d.split_mode != MTK_SPLIT_SERIAL) quarter = {std::max(1, split), 4};
   if (quarter.split) {
     tile = 128;
@@ -452,8 +483,8 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     // other's loads (4095 cubed, f16: 252 us against 566 us on 256x256, one wavefront per SIMD)
     if (d.lda % 2 != 0 || d.ldb % 2 != 0) tile = 128;
   }
-  const int edge = quarter.split ? 64 : tile;  // of a workgroup's tile
-  const int tiles_m = (d.M + edge - 1) / edge, tiles_n = (d.N + edge - 1) / edge;
+  const int rows = quarter.split ? quarter.rows : tile, cols = quarter.split ? 64 : tile;  // of a workgroup's tile
+  const int tiles_m = (d.M + rows - 1) / rows, tiles_n = (d.N + cols - 1) / cols;
   const long long tiles = (long long)tiles_m * tiles_n;
   if (split == 0) {  // fill about one wave of 256 CUs with split-K when the tile grid is small
     split = 1;
@@ -487,7 +518,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   char name[96];
   // operand letters: A [M][K] 'n' / [K][M] 't', B [N][K] 't' / [K][N] 'n'
   snprintf(name, sizeof name, "mtk_gemm_%s_%c%c_%dx%d_%s%s", dt, d.trans_a ? 't' : 'n', d.trans_b ? 't' : 'n', tile,
-           tile, serial ? "s" : direct ? "d" : "v1", !quarter.split ? "" : quarter.waves == 4 ? "q4" : "q");
+           tile, serial ? "s" : direct ? "d" : "v1", !quarter.split ? "" : quarter.rows == 96 ? "q96" : quarter.waves == 4 ? "q4" : "q");
   g.name = name;
   if (quarter.split) g.block = 64u * (unsigned)quarter.waves;
   if (tile == 256 && direct) g.block = 512;  // 256x256 direct-to-LDS tiles run 8 wavefronts
@@ -547,7 +578,9 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
            "gemm %s %s %s M=%d N=%d K=%d tile=%dx%d split_k=%d k_tiles/split=%d k_stagger=%d %s grid=%u%s", dt,
            d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, tile, tile, split, kps,
            a.k_stagger,
-           quarter.split ? "64x64 quarters, K-tiles over the wavefronts" : direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
+           quarter.rows == 96  ? "96x64 workgroups, K-tiles over the wavefronts"
+           : quarter.split     ? "64x64 quarters, K-tiles over the wavefronts"
+           : direct ? "direct-to-LDS" : "2-byte aligned rows", g.grid,
            serial ? " (partitions in sequence per tile, summed in the epilogue)" : split > 1 ? " + splitk_reduce" : "");
   p->description = desc;
   int s = resolve(p);
