@@ -9,7 +9,7 @@
 
 #include <stdint.h>
 
-#define MTK_KARGS_VERSION 14
+#define MTK_KARGS_VERSION 15
 
 /* In-workgroup split-K: bytes of workspace slot per output tile of BM x BM (256 or 128). Each
  * wavefront keeps these accumulator blocks (32 x 32 fp32, 4 KB) of its running sum in the slot,
@@ -31,7 +31,9 @@ typedef struct {
                        else NULL */
   int32_t M, N, K;
   int32_t lda, ldb, ldc;
-  uint32_t a_bytes, b_bytes; /* buffer-resource ranges: loads at or past these byte offsets return 0 */
+  /* buffer-resource ranges: loads at or past these byte offsets return 0 (kernels that take rows at any
+   * 2-byte alignment: counted from the dword in which the operand starts) */
+  uint32_t a_bytes, b_bytes;
   int32_t tiles_m, tiles_n;
   int32_t k_tiles;          /* ceil(K / 64) */
   int32_t k_tiles_per_split;

@@ -144,6 +144,10 @@ struct mtk_plan {
   size_t workspace = 0;
   size_t lt_at = 0, part_kv_at = 0, part_q_at = 0;  // attention backward: byte offsets in the workspace
   size_t part_ml_at = 0;              // byte offset of the per-row pairs in the partial-sum buffer
+  // kernels that read rows at any 2-byte alignment: the operands' exact sizes, from which their buffer
+  // ranges are made when the pointers are known (operand_range)
+  bool any_rows = false;
+  size_t a_exact = 0, b_exact = 0;
   size_t weight_bytes = 0;            // conv: exact byte extent of w (its workspace copy is rounded up)
   bool serial_split = false;          // GEMM split-K run in-workgroup (C written by the main kernel)
   unsigned align_a = 2, align_b = 2;  // required operand alignments (bytes)
@@ -197,6 +201,11 @@ int pow2_vec(std::initializer_list<long long> values) {
 }
 
 bool aligned(const void *p, unsigned a) { return ((uintptr_t)p % a) == 0; }
+
+// Bytes from the dword in which an operand starts to the end of the dword of its last element: the buffer
+// range of kernels that read dwords at any 2-byte alignment. Never a whole dword past the operand, which may
+// be the end of its allocation.
+uint32_t operand_range(const void *p, size_t exact) { return (uint32_t)((exact + ((uintptr_t)p & 2) + 3) & ~(size_t)3); }
 
 float f16_to_f32(uint16_t h) {
   const uint32_t sign = (uint32_t)(h & 0x8000u) << 16, exp = (h >> 10) & 0x1fu, mant = h & 0x3ffu;
@@ -304,11 +313,12 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
     return fail(MTK_ERR_INVALID, "split_mode must be MTK_SPLIT_AUTO, MTK_SPLIT_TWO_PASS or MTK_SPLIT_SERIAL");
   // Buffer ranges end on a whole dword: raw buffer loads range-check per dword, so a last element
   // in the low half of a straddling dword would read as zero. The at most 2 extra bytes lie in the
-  // same aligned dword (same page) as the operand's last element; they are masked in the kernels.
+  // same aligned dword (same page) as the operand's last element; they are masked in the kernels. (For
+  // operands that may start in the middle of a dword: operand_range, once the pointers are known.)
   const uint64_t a_rows = d.trans_a ? d.K : d.M, a_cols = d.trans_a ? d.M : d.K;
-  const uint64_t a_bytes = (((a_rows - 1) * (uint64_t)d.lda + a_cols) * 2 + 3) & ~3ull;
+  const uint64_t a_exact = ((a_rows - 1) * (uint64_t)d.lda + a_cols) * 2, a_bytes = (a_exact + 3) & ~3ull;
   const uint64_t b_rows = d.trans_b ? d.N : d.K, b_cols = d.trans_b ? d.K : d.N;
-  const uint64_t b_bytes = (((b_rows - 1) * (uint64_t)d.ldb + b_cols) * 2 + 3) & ~3ull;
+  const uint64_t b_exact = ((b_rows - 1) * (uint64_t)d.ldb + b_cols) * 2, b_bytes = (b_exact + 3) & ~3ull;
   if (a_bytes > kMaxOperandBytes || b_bytes > kMaxOperandBytes)
     return fail(MTK_ERR_UNSUPPORTED, "operands above 2 GiB are not supported by this build");
 
@@ -455,6 +465,9 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   // Odd leading dimensions: the register-staged kernel, rows at any 2-byte alignment.
   const bool direct = d.lda % 2 == 0 && d.ldb % 2 == 0;
   p->align_a = p->align_b = direct ? 4 : 2;
+  p->any_rows = !direct;
+  p->a_exact = a_exact;
+  p->b_exact = b_exact;
 
   int tile = d.tile;
   int split = d.split_k;
@@ -995,6 +1008,9 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
   if (quarter) {
     g.name = std::string("mtk_conv_f16_gen_128x128_") + (!fast && va == 1 ? "v1q" : "q") + std::to_string(quarter);
     g.block = 64 * quarter;
+    p->any_rows = !fast && va == 1;
+    p->a_exact = x_bytes;
+    p->b_exact = w_bytes;
     a.tiles_m = (int)((M + 63) / 64);
     a.tiles_n = (d.O + 63) / 64;
     set_divisor(a.dOW, ow);
@@ -1228,6 +1244,10 @@ void patch_gemm(const mtk_plan *p, const Launch &l, char *block, const mtk_gemm_
     mtk_tile_args *a = (mtk_tile_args *)block;
     a->A = g->A;
     a->B = g->B;
+    if (p->any_rows) {
+      a->a_bytes = operand_range(g->A, p->a_exact);
+      a->b_bytes = operand_range(g->B, p->b_exact);
+    }
     a->bias = g->bias;
     a->C = two_pass ? nullptr : g->C;
     a->partial = p->workspace ? (float *)ws : nullptr;
@@ -1272,6 +1292,10 @@ int bind_args(const mtk_plan *p, const void *argset, std::vector<Launch> &ls, vo
       mtk_tile_args &a = args_of<mtk_tile_args>(l);
       a.A = c->x;
       a.B = p->workspace ? c->workspace : c->w;
+      if (p->any_rows) {
+        a.a_bytes = operand_range(a.A, p->a_exact);
+        a.b_bytes = operand_range(a.B, p->b_exact);
+      }
       a.bias = c->bias;
       a.C = c->y;
       a.partial = nullptr;

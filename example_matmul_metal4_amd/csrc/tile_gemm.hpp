@@ -92,12 +92,13 @@ __device__ __forceinline__ u32x4 keep_halves(u32x4 v, int n) {
 }
 
 // An operand whose rows are only 2-byte aligned may itself start in the middle of a dword: its
-// buffer starts at that dword, and every offset into it has `mis` (0 or 2) added. kOOBAny lies past
-// any such range.
+// buffer starts at that dword, and every offset into it has `mis` (0 or 2) added. `bytes`, the range from
+// that dword to the end of the last element's, is the host's (operand_range): rounding a size here that
+// was rounded before adding mis would let it end one dword past the operand. kOOBAny lies past any range.
 constexpr uint32_t kOOBAny = 0x80000000u;
 __device__ __forceinline__ rsrc_t make_rsrc_any(const void *p, uint32_t bytes, uint32_t &mis) {
   mis = (uint32_t)(uintptr_t)p & 2u;
-  return make_rsrc((const char *)p - mis, (bytes + mis + 3u) & ~3u);
+  return make_rsrc((const char *)p - mis, bytes);
 }
 
 // ---------------------------------------------------------------- A / B loaders
