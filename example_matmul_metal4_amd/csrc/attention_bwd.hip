@@ -150,7 +150,7 @@ __device__ __forceinline__ void attn_bwd_pre(const mtk_attn_bwd_kargs &a) {
 // Steps [i0, i1) of a walk of n steps for workgroup `part` of those that share it (n > 0), and how many
 // do; part >= that count has none.
 __device__ __forceinline__ int walk_part(int n, int cap, int part, int &i0, int &i1) {
-  const int parts = max(1, (n + cap - 1) / cap);
+  const int parts = n <= cap ? 1 : (n - 1) / cap + 1;
   const int per = (n + parts - 1) / parts;
   i0 = min(n, part * per);
   i1 = min(n, i0 + per);

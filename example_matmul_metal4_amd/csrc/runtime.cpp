@@ -619,12 +619,14 @@ struct WalkShare {
 WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal, double step_us, double elems, double sum_us,
                       int cus) {
   const int longest = *std::max_element(walks.begin(), walks.end());
+  // (w + cap - 1) / cap would overflow for the cap of walks that nothing shares, INT32_MAX
+  auto shares = [](int w, int cap) { return w <= cap ? 1 : (w - 1) / cap + 1; };
   auto expected = [&](int cap) {
     double total = 0, shared = 0;
     long long n = 0;
     int item = 0;
     for (int w : walks) {
-      const int parts = std::max(1, (w + cap - 1) / cap);
+      const int parts = shares(w, cap);
       total += (double)w * count;
       n += parts * count;
       item = std::max(item, (w + parts - 1) / parts);
@@ -648,7 +650,10 @@ WalkShare share_walks(const std::vector<int> &walks, long long count, bool equal
     }
   }
   if (best.parts > 1 && walks.size() <= 64) {
-    auto share = [&](int w) { return best.cap >= w ? w : (w + (w + best.cap - 1) / best.cap - 1) / ((w + best.cap - 1) / best.cap); };
+    auto share = [&](int w) {
+      const int parts = shares(w, best.cap);
+      return (w + parts - 1) / parts;
+    };
     for (size_t i = 0; i < walks.size(); ++i) best.order[i] = (uint8_t)i;
     std::stable_sort(best.order, best.order + walks.size(),
                      [&](uint8_t x, uint8_t y) { return share(walks[x]) > share(walks[y]); });

@@ -1,6 +1,7 @@
 """The host runtime (csrc/runtime.cpp) built with AddressSanitizer and UndefinedBehaviorSanitizer
 runs the C-ABI tests that need no GPU (tests/test_abi.py: descriptor validation, kernel-select of
-dry plans, describe / work / destroy, validate, the no-device path) without a sanitizer report.
+dry plans, describe / work / destroy, validate, the no-device path) and the planner tests that stand
+beside the GPU tests (every dispatch rule, long shared walks among them) without a sanitizer report.
 Host code only: the library's device part (the scratch object) is linked unchanged."""
 import os
 import shutil
@@ -11,6 +12,10 @@ import pytest
 
 import example_matmul_metal4_amd as mtk
 
+#: files with tests of the planner alone
+PLANNED = ["test_abi", "test_attention_bwd_shared_gpu", "test_attention_kv_gpu", "test_attention_plan_sweep_gpu",
+           "test_attention_bwd_plan_sweep_gpu", "test_conv_plan_sweep_gpu", "test_conv_quarter_gpu", "test_gemm_plan_sweep_gpu",
+           "test_gemm_quarter_gpu", "test_gemm_tall_gpu"]
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
@@ -40,8 +45,8 @@ def test_dry_plan_abi_tests_under_asan_and_ubsan(tmp_path):
              "print(any(l.rstrip().endswith(m.LIB_PATH) for l in open('/proc/self/maps')))")
     r = subprocess.run([sys.executable, "-c", probe], env=env, capture_output=True, text=True, cwd=ROOT, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "True", r.stdout + r.stderr
-    r = subprocess.run([sys.executable, "-m", "pytest", "-q", "-p", "no:cacheprovider", "-m", "not gpu",
-                        os.path.join(ROOT, "tests", "test_abi.py")],
+    r = subprocess.run([sys.executable, "-m", "pytest", "-q", "-p", "no:cacheprovider", "-m", "not gpu"] +
+                       [os.path.join(ROOT, "tests", f + ".py") for f in PLANNED],
                        env=env, capture_output=True, text=True, cwd=ROOT, timeout=600)
     out = r.stdout + r.stderr
     assert r.returncode == 0, out[-4000:]
