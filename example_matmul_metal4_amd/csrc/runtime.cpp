@@ -472,14 +472,22 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   int tile = d.tile;
   int split = d.split_k;
   // Quarter tiles: only where neither a tile, a partition layout nor a schedule is asked for; and for A
-  // [K][M] with odd rows of B always (no other kernel reads them).
+  // [K][M] with odd rows of B always, as no other kernel reads them: a requested tile, or partitions run
+  // in sequence, is refused there.
+  if (d.trans_a && !direct) {
+    const char *what = d.tile != 0 ? "a tile" : d.split_mode == MTK_SPLIT_SERIAL && split != 1 && k_tiles > 1 ? "in-workgroup split-K" : nullptr;
+    if (what) {
+      delete p;
+      return fail(MTK_ERR_UNSUPPORTED, "A [K][M] with odd rows of B (ldb %d) runs on 64x64 workgroups: %s cannot be chosen", d.ldb, what);
+    }
+  }
   Quarter quarter;
   if (tile == 0 && d.split_mode == MTK_SPLIT_AUTO && d.k_stagger == 0 && split <= 1) {
     const int cus = ctx ? ctx->prop.multiProcessorCount : 256;
     if (direct && !d.trans_a) quarter = tall_plan(d.M, d.N, k_tiles, split, d.trans_b, cus);
     if (!quarter.split) quarter = quarter_plan(d.M, d.N, k_tiles, split, direct, cus);
   }
-  if (d.trans_a && !direct && !quarter.split && d.split_mode != MTK_SPLIT_SERIAL) quarter = {std::max(1, split), 4};
+  if (d.trans_a && !direct && !quarter.split) quarter = {std::max(1, split), 4};
   if (quarter.split) {
     tile = 128;
     split = quarter.split;

@@ -107,6 +107,8 @@ int mtk_set_stream(mtk_ctx *ctx, void *hip_stream);
  * with the bias added last (the reference's reduce_sum_2, matmul.swift:298-311, 451-474, without
  * its in-place race); 0 = let the plan choose.
  * tile: 0 = let the plan choose; else 128 or 256 (square MFMA workgroup tile).
+ * A [K][lda] with an odd ldb runs on 64x64 workgroups only: MTK_ERR_UNSUPPORTED for a tile, and for
+ * MTK_SPLIT_SERIAL unless there is one partition.
  * split_mode (split_k > 1): how the partitions are scheduled; for one partition layout the
  * arithmetic, and so the result, is the same bit for bit:
  *   MTK_SPLIT_AUTO     in-workgroup when the tile grid fills the device and split_k <= 4,

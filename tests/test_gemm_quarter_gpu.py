@@ -68,3 +68,22 @@ def test_quarter_tiles(dev, case):
     # one rounding to the output type, fp32 sums of K products in any order on either side
     bound = oracle.ulp(exp, dtype) + 2 * K * 2.0 ** -24 * (a @ (b.T if tb else b) + np.abs(oracle.to_f32(bias, dtype)))
     assert np.all(np.isfinite(got)) and np.all(np.abs(got - exp) <= bound), np.abs(got - exp).max()
+
+
+def _odd_t(split_k=1, **kw):
+    return mtk.GemmPlan(None, 300, 64, 71, trans_a=True, split_k=split_k, **kw)  # B [64][71]: odd rows
+
+
+def test_transposed_a_with_odd_rows_is_planned_or_refused():
+    # CPU: only the quarter kernels read A [K][M] beside odd rows of B, so every accepted plan names one of
+    # them (a kernel that is compiled); a tile or an in-workgroup schedule that they cannot honour is refused
+    for plan in (_odd_t(), _odd_t(0), _odd_t(2), _odd_t(split_mode="two_pass"), _odd_t(split_mode="serial"),
+                 _odd_t(3, split_mode="two_pass", k_stagger=2),
+                 mtk.GemmPlan(None, 300, 63, 60, trans_a=True, trans_b=False, split_k=4, split_mode="serial"),  # one K-tile
+                 mtk.GemmPlan(None, 4096, 4095, 8192, trans_a=True, trans_b=False, split_k=0)):
+        assert "_128x128_v1q" in plan.describe(), plan.describe()
+    for kw in (dict(tile=256), dict(tile=128), dict(tile=256, split_mode="serial"), dict(split_k=2, split_mode="serial"),
+               dict(split_k=0, split_mode="serial")):
+        with pytest.raises(mtk.MtkError) as e:
+            _odd_t(**kw)
+        assert e.value.status == mtk.MTK_ERR_UNSUPPORTED, kw
