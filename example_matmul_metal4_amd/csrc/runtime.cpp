@@ -597,7 +597,7 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   char desc[320];
   snprintf(desc, sizeof desc,
            "gemm %s %s %s M=%d N=%d K=%d tile=%dx%d split_k=%d k_tiles/split=%d k_stagger=%d %s grid=%u%s", dt,
-           d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, tile, tile, split, kps,
+           d.trans_a ? "A[K][M]" : "A[M][K]", d.trans_b ? "B[N][K]" : "B[K][N]", d.M, d.N, d.K, rows, cols, split, kps,
            a.k_stagger,
            quarter.rows == 96  ? "96x64 workgroups, K-tiles over the wavefronts"
            : quarter.split     ? "64x64 quarters, K-tiles over the wavefronts"
@@ -1041,7 +1041,7 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
              (oidhw ? 2.0 * (double)w_bytes : 0.0);  // the re-layout reads and writes the weights once
   char desc[288];
   snprintf(desc, sizeof desc, "conv%dd f16 implicit-GEMM M=%lld N=%d K=%lld out=%dx%dx%d tile=%dx%d gather=%s grid=%u%s",
-           d.rank, M, d.O, K, od, oh, ow, quarter ? 64 : bm, quarter ? 64 : bn, kind, g.grid,
+           d.rank, M, d.O, K, od, oh, ow, quarter ? 64 : bm, quarter ? 64 : bn, quarter ? "gen" : kind, g.grid,
            oidhw ? " weights OIDHW (re-laid out in the workspace)" : "");
   p->description = desc;
   s = resolve(p);

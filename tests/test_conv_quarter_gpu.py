@@ -9,6 +9,7 @@ import oracle
 from oracle import generators as gen
 
 from test_conv_gpu import _bit_exact, _run
+from test_gemm_quarter_gpu import _tile_and_grid
 
 C2, C3 = oracle.ConvDims.conv2d, oracle.ConvDims.conv3d
 # rank, dims, kernel: edges of the 64-pixel and 64-channel tiles, channels whose chunks share a K-tile with
@@ -32,7 +33,9 @@ def _plan(dev, rank, dims, **kw):
 def test_which_plans_are_quartered():
     # CPU: the planner alone
     for rank, dims, kern in CASES:
-        assert _plan(None, rank, dims).describe().endswith("_" + kern), (dims.as_dict(), _plan(None, rank, dims).describe())
+        text = _plan(None, rank, dims).describe()
+        assert text.endswith("_" + kern) and " gather=gen " in text, (dims.as_dict(), text)
+        _tile_and_grid(text, dims.N * dims.OD * dims.OH * dims.OW, dims.O, 64, 64)
     for dims in (C2(N=1, H=40, W=40, C=12, O=16), C2(N=1, H=40, W=40, C=16, O=16, KH=11, KW=3), C2(N=1, H=40, W=40, C=64, O=64, KH=1, KW=1),
                  C2(N=8, H=128, W=128, C=256, O=256), C2(N=4, H=100, W=100, C=96, O=256)):
         assert not _plan(None, 2, dims).describe().rsplit("_", 1)[1].lstrip("v1").startswith("q"), _plan(None, 2, dims).describe()

@@ -28,11 +28,19 @@ def _plan(dev, case):
                         lda=(M if ta else K) + pa, ldb=(K if tb else N) + pb)
 
 
+def _tile_and_grid(text, M, N, rows, cols):
+    """The description's tile and grid are the workgroups that run."""
+    word = lambda key: text.split(f" {key}=")[1].split()[0]
+    assert word("tile") == f"{rows}x{cols}", text
+    assert int(word("grid")) == -(-M // rows) * -(-N // cols) * int(word("split_k") if " split_k=" in text else 1), text
+
+
 def test_which_plans_are_quartered():
     # CPU: the planner alone
     for c in CASES:
         kern = _plan(None, c).describe().split("kernels: ")[1].split()[0]
         assert kern.endswith("q4" if c in FOUR else "q"), (c, kern)
+        _tile_and_grid(_plan(None, c).describe(), c[0], c[1], 64, 64)
     assert "splitk_reduce" in _plan(None, CASES[20]).describe() and "splitk_reduce" in _plan(None, CASES[22]).describe()
     # larger grids, requested tiles, partitions or schedules, and K of fewer than four K-tiles are not
     for kw in (dict(M=2048, N=2048, K=512), dict(M=1024, N=1024, K=1024, tile=128), dict(M=512, N=512, K=4096, split_k=4),

@@ -5,7 +5,7 @@ import pytest
 
 import example_matmul_metal4_amd as mtk
 
-from test_gemm_quarter_gpu import _plan, test_quarter_tiles as _check
+from test_gemm_quarter_gpu import _plan, _tile_and_grid, test_quarter_tiles as _check
 
 # M, N, K, trans_a, trans_b, padding of A's and B's rows, split_k, dtype
 CASES = [(65, 16383, 1026, False, True, 0, 0, 1, "f16"), (96, 10946, 1032, False, False, 2, 4, 1, "bf16"),
@@ -18,6 +18,7 @@ def test_which_plans_are_tall():
     # CPU: the planner alone
     for c in CASES:
         assert "q96" in _plan(None, c).describe(), (c, _plan(None, c).describe())
+        _tile_and_grid(_plan(None, c).describe(), c[0], c[1], 96, 64)
     assert "splitk_reduce" in _plan(None, CASES[2]).describe() and "splitk_reduce" in _plan(None, CASES[7]).describe()
     # other row counts, odd rows, transposed A, requested tiles or partitions, short K, few columns are not
     for kw in (dict(M=64), dict(M=97), dict(M=193), dict(K=2049), dict(trans_a=True), dict(tile=128), dict(split_k=4),
