@@ -9,7 +9,7 @@
 
 #include <stdint.h>
 
-#define MTK_KARGS_VERSION 15
+#define MTK_KARGS_VERSION 16
 
 /* In-workgroup split-K: bytes of workspace slot per output tile of BM x BM (256 or 128). Each
  * wavefront keeps these accumulator blocks (32 x 32 fp32, 4 KB) of its running sum in the slot,
@@ -106,9 +106,9 @@ typedef struct {
   int32_t H_kv; /* K/V heads (divides H): query head h reads K/V head h / (H / H_kv) */
   int32_t D;    /* head dimension */
   /* key-split kernels (q_blocks: blocks of 32 (query, query head) rows of one K/V head): */
-  int32_t kv_splits; /* workgroups that share the keys of one row block (>= 1) */
+  int32_t kv_splits; /* parts of the keys of one row block (>= 1), one workgroup each or walked in turn */
   int32_t part_ld;   /* floats per row of part */
-  float *part;       /* kv_splits > 1: [B * H_kv][q_blocks][kv_splits][32][part_ld] weighted V sums */
+  float *part;       /* shared splits: [B * H_kv][q_blocks][kv_splits][32][part_ld] weighted V sums */
   float *part_ml;    /* ... and per row (exponent offset in log2, sum of weights) */
 } mtk_attn_kargs;
 

@@ -138,7 +138,8 @@ struct mtk_plan {
   mtk_permute_desc perm{};
   std::vector<Launch> launches;
   // attention with the keys split over workgroups: `launches` need a partial-sum buffer of the
-  // library's; `plain` is the plan without one (one kernel), run where there is none
+  // library's; `plain` is the plan without one (one kernel that walks the splits in turn, the same bits),
+  // run where there is none
   bool needs_part = false;
   std::vector<Launch> plain;
   size_t workspace = 0;
@@ -1140,9 +1141,10 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
     // against 15.1, 64 x 4096, B 1: 23 -> 19)
     int splits = (int)std::min<long long>(cus / std::max<long long>(wgs, 1), key_tiles / 8);
     if (splits < 2 || key_tiles < ((long long)d.B * d.H * d.S_q <= 512 ? 48 : 96)) splits = 1;
-    auto kv_launch = [&](int n, int sp) {
+    auto kv_launch = [&](int n, bool shared) {  // shared: one workgroup per split of the keys
       Launch l;
-      l.name = "mtk_attn_kv_d" + std::to_string(dp) + "_" + std::to_string(n) + (d.dtype == MTK_F16 ? "_f16" : "_bf16");
+      l.name = "mtk_attn_kv_d" + std::to_string(dp) + "_" + std::to_string(n) + (splits > 1 && !shared ? "_seq" : "") +
+               (d.dtype == MTK_F16 ? "_f16" : "_bf16");
       l.block = dp == 256 ? 256 : 512;
       mtk_attn_kargs a{};
       a.B = d.B;
@@ -1156,9 +1158,9 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
       a.q_bytes = (uint32_t)q_bytes;
       a.kv_bytes = (uint32_t)kv_bytes;
       a.D = d.D;
-      a.kv_splits = sp;
+      a.kv_splits = splits;
       a.part_ld = (blocks32 + n - 1) / n * n * 32;
-      l.grid = (unsigned)(units * ((blocks32 + n - 1) / n) * sp);
+      l.grid = (unsigned)(units * ((blocks32 + n - 1) / n) * (shared ? splits : 1));
       set_args(l, a);
       return l;
     };
@@ -1169,15 +1171,15 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
     if (splits > 1) {
       p->needs_part = true;
       p->part_ml_at = ml_at;
-      p->plain.push_back(kv_launch(ndb, 1));
-      p->launches.push_back(kv_launch(full, splits));
+      p->plain.push_back(kv_launch(ndb, false));
+      p->launches.push_back(kv_launch(full, true));
       Launch c = p->launches[0];
       c.name = std::string("mtk_attn_kv_combine_") + (d.dtype == MTK_F16 ? "f16" : "bf16");
       c.block = 256;
       c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 8) + 255) / 256);
       p->launches.push_back(c);
     } else {
-      p->launches.push_back(kv_launch(ndb, 1));
+      p->launches.push_back(kv_launch(ndb, false));
     }
     rows = 32;
   }

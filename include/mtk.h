@@ -195,7 +195,7 @@ int mtk_gemm_run_noalloc(const mtk_plan *plan, const mtk_gemm_args *args);
  * wavefronts and, behind a long cache, over workgroups (sums in a fixed order, reproducible, but not
  * the order of the 128-row kernel). The latter keep partial sums in a 16 MiB buffer of the context,
  * allocated once, for work on the context's own stream, and in one of the graph's for mtk_graph_*; on
- * an external stream or inside a caller's stream capture the keys stay in one workgroup. */
+ * an external stream or inside a caller's stream capture one workgroup walks the parts of the keys (same bits). */
 #define MTK_ATTN_MAX_HEAD_DIM 512
 
 typedef struct {

@@ -76,17 +76,18 @@ def test_key_split_parity(dev, case):
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", SPLIT, ids=str)
 def test_split_keys_in_graphs_and_on_other_streams(dev, case):
-    # a graph has partial sums of its own (same kernels, same bits as an eager call); work on a stream
-    # that is not the context's own takes the one-kernel plan, which sums in another order
+    # the same bits from an eager call, from a graph (which has partial sums of its own), on a stream that is
+    # not the context's own and in a caller's capture of one (where one workgroup walks the splits)
     B, H, Hkv, Sq, Skv, D, causal, dtype = case
     plan = _plan(dev, case)
     Q, K, V = _inputs(case)
     bufs = [dev.upload(x) for x in (Q, K, V)]
     outs = [dev.empty(Q.nbytes) for _ in range(3)]
+    lses = [dev.empty(4 * B * H * Sq) for _ in range(2)]
     read = lambda o: dev.download(o, Q.shape, np.uint16)
-    plan.run(*bufs, outs[0])
+    plan.run(*bufs, outs[0], lses[0])
     dev.sync()
-    ref = read(outs[0])
+    ref, ref_lse = read(outs[0]), dev.download(lses[0], (B, H, Sq), np.uint32)
     g = plan.graph([plan.args(*bufs, outs[1])], steps=3)
     try:
         for _ in range(3):
@@ -100,15 +101,30 @@ def test_split_keys_in_graphs_and_on_other_streams(dev, case):
     hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library has loaded
     stream = ctypes.c_void_p()
     assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0  # non-blocking
+    graph, graph_exec = ctypes.c_void_p(), ctypes.c_void_p()
+    poison = lambda: (dev.upload_into(outs[2], np.full(Q.shape, 0x7E00, np.uint16)),
+                      dev.upload_into(lses[1], np.zeros((B, H, Sq), np.uint32)))
+    same = lambda: (np.array_equal(read(outs[2]), ref) and
+                    np.array_equal(dev.download(lses[1], (B, H, Sq), np.uint32), ref_lse))
     mtk._check(mtk.lib().mtk_set_stream(dev.handle, stream))
     try:
-        plan.run(*bufs, outs[2])
+        poison()
+        plan.run(*bufs, outs[2], lses[1])
         dev.sync()
+        assert same(), "another stream"
+        assert hip.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+        plan.run(*bufs, outs[2], lses[1])
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(graph_exec), graph, None, None, ctypes.c_size_t(0)) == 0
+        for _ in range(3):
+            poison()
+            assert hip.hipGraphLaunch(graph_exec, stream) == 0
+            dev.sync()
+            assert same(), "a captured call"
     finally:
         mtk._check(mtk.lib().mtk_set_stream(dev.handle, None))
-        hip.hipStreamDestroy(stream)
-    got = oracle.to_f32(read(outs[2]).view(Q.dtype), dtype).astype(np.float64)
-    exp = oracle.to_f32(ref.view(Q.dtype), dtype).astype(np.float64)
-    assert oracle.rel_frobenius(got, exp) <= (1e-3 if dtype == "f16" else 8e-3)  # two roundings of the output
-    for x in bufs + outs:
+        for destroy, x in (("hipGraphExecDestroy", graph_exec), ("hipGraphDestroy", graph), ("hipStreamDestroy", stream)):
+            if x:
+                getattr(hip, destroy)(x)
+    for x in bufs + outs + lses:
         x.free()
