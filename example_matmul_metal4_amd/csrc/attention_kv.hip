@@ -344,17 +344,16 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
   KvSum total;
   constexpr int kAhead = 8;  // splits whose partials are in flight at once
   for (int s0 = 0; s0 < S; s0 += kAhead) {
-    KvSum t[kAhead];
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      if (s0 + i >= S) break;
-      const f32x2 e = *(const f32x2 *)(ml + (size_t)(s0 + i) * 2 * kKvRows);
-      const float *p = x + (size_t)(s0 + i) * kKvRows * a.part_ld;
-      t[i] = KvSum{e.x, e.y, *(const f32x4 *)p, *(const f32x4 *)(p + 4)};
-    }
+    KvSum t[kAhead];  // past the last split: no keys, which add nothing
 #pragma unroll
     for (int i = 0; i < kAhead; ++i)
-      if (s0 + i < S) add_keys(total, t[i]);
+      if (s0 + i < S) {
+        const f32x2 e = *(const f32x2 *)(ml + (size_t)(s0 + i) * 2 * kKvRows);
+        const float *p = x + (size_t)(s0 + i) * kKvRows * a.part_ld;
+        t[i] = KvSum{e.x, e.y, *(const f32x4 *)p, *(const f32x4 *)(p + 4)};
+      }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) add_keys(total, t[i]);
   }
   const int q = rr / G;
   store_row<DT>(a, b, q, hk * G + (rr - q * G), 8 * ch, total, ch == 0);

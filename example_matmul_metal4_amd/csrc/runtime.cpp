@@ -52,7 +52,6 @@ int fail(int status, const char *fmt, ...) {
 constexpr uint64_t kMaxOperandBytes = (1ull << 31) - 256;  // buffer-resource ranges (see device.hpp)
 constexpr int kAutoKStagger = 16;  // in-workgroup split-K: boundary offsets span up to 16 K-tiles
 constexpr int kMaxHeadDim = MTK_ATTN_MAX_HEAD_DIM;  // largest padded head dimension compiled (512)
-constexpr size_t kPartBytes = 16u << 20;  // partial-sum buffer of a context or graph (attention, keys split)
 
 }  // namespace
 
@@ -63,35 +62,83 @@ struct mtk_ctx {
   hipStream_t stream = nullptr;
   std::vector<hipModule_t> modules;
   std::map<std::string, hipFunction_t> functions;
-  // Partial sums of attention plans that split the keys over workgroups. One buffer for the context's
-  // own stream, whose kernels use it one after another; part_mu is held while a plan enqueues its
-  // kernels, so that two threads' kernels do not interleave on it.
+  // Partial sums of attention plans that split the keys over workgroups: kParts regions of one
+  // allocation, made with the first such plan (no launch allocates) and freed with the context. Region 0
+  // is the own stream's, whose kernels use it one after another; others go to the first external streams and
+  // to the first captures of a caller (one per stream of a capture, whose graph may be replayed at any
+  // later time) and stay theirs. A call that finds no region walks the splits in one workgroup, with the
+  // same result. part_mu is held from the choice of a region until the kernels are enqueued, so that two
+  // threads' do not interleave on it.
+  struct Part {
+    hipStream_t stream = nullptr;
+    unsigned long long capture = 0;  // id of the capture, 0: none
+    hipEvent_t done = nullptr;       // behind the last use by an external stream
+  };
+  static constexpr int kParts = 32, kCaptures = 16;  // captures have regions from kCaptures on
   std::mutex part_mu;
-  void *part = nullptr;
+  char *parts = nullptr;
+  Part part[kParts];
 
-  // That buffer, or NULL when there is none to be had: work goes to an external stream (which this
-  // context cannot order against its own), the stream is being captured (the graph could replay next
-  // to later work) or the allocation fails. The caller holds part_mu.
-  void *part_buffer() {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusActive;
-    if (stream != own_stream || hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
-      return nullptr;
-    if (!part) part = alloc_part();
-    return part;
-  }
+  // Bytes of a region: two or more splits are taken while their workgroups are no more than the CUs, and each
+  // writes 32 rows of at most 128 sums and two values per row.
+  size_t part_capacity() const { return (size_t)prop.multiProcessorCount * 32 * (128 + 2) * sizeof(float); }
 
-  static void *alloc_part() {
-    // relaxed: another thread's stream capture does not make this allocation an error
+  // The calls below may meet another thread's stream capture, which they neither disturb nor fail for.
+  struct Relaxed {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+    const bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~Relaxed() {
+      if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+  };
+  static void *alloc_part(size_t bytes) {
+    Relaxed relaxed;
     void *buf = nullptr;
-    if (hipMalloc(&buf, kPartBytes) != hipSuccess) {
+    if (hipMalloc(&buf, bytes) != hipSuccess) {
       buf = nullptr;
       (void)hipGetLastError();
     }
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
     return buf;
   }
+  static void free_part(void *buf) {  // waits for the device
+    Relaxed relaxed;
+    (void)hipFree(buf);
+  }
+
+  // The region for work on the current stream, or -1. The caller holds part_mu.
+  int take_part() {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (!parts) return -1;
+    if (hipStreamGetCaptureInfo(stream, &cs, &id) != hipSuccess || cs == hipStreamCaptureStatusInvalidated) return -1;
+    if (cs == hipStreamCaptureStatusNone) id = 0;
+    if (stream == own_stream && !id) return 0;
+    // No event is asked about or waited for that another stream has recorded: where that stream is being
+    // captured by now, the question would break its capture.
+    for (int i = id ? kCaptures : 1; i < (id ? kParts : kCaptures); ++i) {
+      Part &r = part[i];
+      if (r.stream && (r.stream != stream || r.capture != id)) continue;
+      if (!id) {
+        // A stream's first use creates the event; at a later one the handle may be another stream's by now,
+        // the last one's work still running.
+        const hipError_t e = r.stream ? hipStreamWaitEvent(stream, r.done, 0) : hipEventCreateWithFlags(&r.done, hipEventDisableTiming);
+        if (e != hipSuccess) {
+          (void)hipGetLastError();
+          return -1;
+        }
+      }
+      r.stream = stream;
+      r.capture = id;
+      return i;
+    }
+    return -1;
+  }
+  // Work on region i (or none) has been enqueued.
+  int leave_part(int i) {
+    if (i > 0 && i < kCaptures) HIP_TRY(hipEventRecord(part[i].done, part[i].stream));
+    return MTK_OK;
+  }
+  void *part_at(int i) { return parts + i * part_capacity(); }
 
   int function(const std::string &name, hipFunction_t *f) {
     auto it = functions.find(name);
@@ -144,7 +191,7 @@ struct mtk_plan {
   std::vector<Launch> plain;
   size_t workspace = 0;
   size_t lt_at = 0, part_kv_at = 0, part_q_at = 0;  // attention backward: byte offsets in the workspace
-  size_t part_ml_at = 0;              // byte offset of the per-row pairs in the partial-sum buffer
+  size_t part_ml_at = 0, part_bytes = 0;  // the per-row pairs' offset in the partial-sum buffer, its size
   // kernels that read rows at any 2-byte alignment: the operands' exact sizes, from which their buffer
   // ranges are made when the pointers are known (operand_range)
   bool any_rows = false;
@@ -1167,10 +1214,14 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
     // partial sums, then the rows' (exponent offset, weight sum) pairs
     const size_t part_rows = (size_t)units * splits * 32;
     const size_t ml_at = part_rows * ((blocks32 + full - 1) / full * full * 32) * sizeof(float);
-    if (ml_at + part_rows * 8 > kPartBytes) splits = 1;
     if (splits > 1) {
       p->needs_part = true;
+      if (ctx && hipSetDevice(ctx->device) == hipSuccess) {
+        std::lock_guard<std::mutex> lock(ctx->part_mu);
+        if (!ctx->parts) ctx->parts = (char *)mtk_ctx::alloc_part(mtk_ctx::kParts * ctx->part_capacity());
+      }
       p->part_ml_at = ml_at;
+      p->part_bytes = ml_at + part_rows * 8;
       p->plain.push_back(kv_launch(ndb, false));
       p->launches.push_back(kv_launch(full, true));
       Launch c = p->launches[0];
@@ -1387,20 +1438,38 @@ size_t argset_size(const mtk_plan *p) {
   }
 }
 
+// The partial-sum region of a plan that needs one, from its choice until the kernels are enqueued.
+struct PartUse {
+  mtk_ctx *ctx = nullptr;
+  std::unique_lock<std::mutex> lock;
+  int region = -1;
+  void *buf = nullptr;
+
+  explicit PartUse(const mtk_plan *p) {
+    if (!p->needs_part) return;
+    ctx = p->ctx;
+    lock = std::unique_lock<std::mutex>(ctx->part_mu);
+    region = ctx->take_part();
+    if (region >= 0) buf = ctx->part_at(region);
+  }
+  int leave() {
+    const int i = region;
+    region = -1;
+    return i >= 0 ? ctx->leave_part(i) : MTK_OK;
+  }
+  ~PartUse() { (void)leave(); }
+};
+
 int run_plan(const mtk_plan *p, const void *argset) {
   if (!p) return fail(MTK_ERR_INVALID, "null plan");
   if (!p->ctx) return fail(MTK_ERR_INVALID, "plan was created without a context (dry plan)");
   HIP_TRY(hipSetDevice(p->ctx->device));
-  std::unique_lock<std::mutex> lock(p->ctx->part_mu, std::defer_lock);
-  void *part = nullptr;
-  if (p->needs_part) {
-    lock.lock();
-    part = p->ctx->part_buffer();
-  }
+  PartUse part(p);
   std::vector<Launch> ls;
-  int s = bind_args(p, argset, ls, part);
-  if (s != MTK_OK) return s;
-  return launch_all(p, ls, nullptr);
+  int s = bind_args(p, argset, ls, part.buf);
+  if (s == MTK_OK) s = launch_all(p, ls, nullptr);
+  const int left = part.leave();
+  return s != MTK_OK ? s : left;
 }
 
 std::string self_dir() {
@@ -1530,7 +1599,9 @@ int mtk_destroy(mtk_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->own_stream);
     (void)hipStreamDestroy(ctx->own_stream);
   }
-  if (ctx->part) (void)hipFree(ctx->part);
+  if (ctx->parts) mtk_ctx::free_part(ctx->parts);
+  for (auto &r : ctx->part)
+    if (r.done) (void)hipEventDestroy(r.done);
   for (hipModule_t m : ctx->modules) (void)hipModuleUnload(m);
   delete ctx;
   return MTK_OK;
@@ -1608,6 +1679,7 @@ int mtk_sync(mtk_ctx *ctx) {
 
 int mtk_set_stream(mtk_ctx *ctx, void *hip_stream) {
   if (!ctx) return fail(MTK_ERR_INVALID, "null context");
+  std::lock_guard<std::mutex> lock(ctx->part_mu);  // not between a region's choice and its kernels
   ctx->stream = hip_stream ? (hipStream_t)hip_stream : ctx->own_stream;
   return MTK_OK;
 }
@@ -1725,9 +1797,9 @@ int mtk_graph_create(const mtk_plan *p, const void *arg_sets, int nsets, int ste
   struct Part {  // given to the graph at the end, freed on every earlier return
     void *buf;
     ~Part() {
-      if (buf) (void)hipFree(buf);
+      if (buf) mtk_ctx::free_part(buf);
     }
-  } part{p->needs_part ? mtk_ctx::alloc_part() : nullptr};
+  } part{p->needs_part ? mtk_ctx::alloc_part(p->part_bytes) : nullptr};
   std::vector<std::vector<Launch>> bound((size_t)nsets);
   for (int i = 0; i < nsets; ++i) {
     int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i], part.buf);
@@ -1785,7 +1857,7 @@ int mtk_graph_destroy(mtk_graph *g) {
   if (!g) return MTK_OK;
   if (g->exec) (void)hipGraphExecDestroy(g->exec);
   if (g->graph) (void)hipGraphDestroy(g->graph);
-  if (g->part) (void)hipFree(g->part);  // waits for the device
+  if (g->part) mtk_ctx::free_part(g->part);
   delete g;
   return MTK_OK;
 }
@@ -1798,15 +1870,10 @@ int mtk_profile(const mtk_plan *p, const void *arg_sets, int nsets, int warmup, 
   memset(out, 0, sizeof *out);
   const size_t stride = argset_size(p);
   HIP_TRY(hipSetDevice(p->ctx->device));
-  std::unique_lock<std::mutex> lock(p->ctx->part_mu, std::defer_lock);
-  void *part = nullptr;
-  if (p->needs_part) {
-    lock.lock();
-    part = p->ctx->part_buffer();
-  }
+  PartUse part(p);
   std::vector<std::vector<Launch>> bound((size_t)nsets);
   for (int i = 0; i < nsets; ++i) {
-    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i], part);
+    int s = bind_args(p, (const char *)arg_sets + stride * i, bound[(size_t)i], part.buf);
     if (s != MTK_OK) return s;
   }
   for (int i = 0; i < warmup; ++i) {

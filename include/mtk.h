@@ -193,9 +193,12 @@ int mtk_gemm_run_noalloc(const mtk_plan *plan, const mtk_gemm_args *args);
  * softmax blocks, one workgroup per CU; D = 128 or 64 only). Same results bit for bit. With 0, calls
  * with few queries or one short sequence (D % 8 == 0, up to 256) run kernels that split the keys over
  * wavefronts and, behind a long cache, over workgroups (sums in a fixed order, reproducible, but not
- * the order of the 128-row kernel). The latter keep partial sums in a 16 MiB buffer of the context,
- * allocated once, for work on the context's own stream, and in one of the graph's for mtk_graph_*; on
- * an external stream or inside a caller's stream capture one workgroup walks the parts of the keys (same bits). */
+ * the order of the 128-row kernel). The latter keep partial sums in a buffer of the context: 130 MiB in 32
+ * regions, allocated with the first such plan and freed with the context. The context's own stream has
+ * one, the first 15 external streams and the first 16 captures of a caller (each stream of one counts)
+ * have one each until then. A graph of mtk_graph_create has partial sums of its own, freed with it. With
+ * no region left, or no memory for them, one workgroup walks the parts of the keys: the same result bit
+ * for bit, but slower. */
 #define MTK_ATTN_MAX_HEAD_DIM 512
 
 typedef struct {

@@ -2,6 +2,7 @@
 few queries, or one short sequence. Whole outputs against the CPU oracle (Network.swift:134-179,
 286-311) with the acceptance of test_attention_gpu.check; the row log-sum-exp against float64."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -77,7 +78,7 @@ def test_key_split_parity(dev, case):
 @pytest.mark.parametrize("case", SPLIT, ids=str)
 def test_split_keys_in_graphs_and_on_other_streams(dev, case):
     # the same bits from an eager call, from a graph (which has partial sums of its own), on a stream that is
-    # not the context's own and in a caller's capture of one (where one workgroup walks the splits)
+    # not the context's own and in a caller's capture of one
     B, H, Hkv, Sq, Skv, D, causal, dtype = case
     plan = _plan(dev, case)
     Q, K, V = _inputs(case)
@@ -128,3 +129,162 @@ def test_split_keys_in_graphs_and_on_other_streams(dev, case):
                 getattr(hip, destroy)(x)
     for x in bufs + outs + lses:
         x.free()
+
+
+def _hip():
+    return ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library has loaded
+
+
+class _Stream:
+    """A non-blocking stream of the caller's, current in the context while entered."""
+
+    def __init__(self, dev):
+        self.dev, self.handle = dev, ctypes.c_void_p()
+        assert _hip().hipStreamCreateWithFlags(ctypes.byref(self.handle), 1) == 0
+
+    def __enter__(self):
+        mtk._check(mtk.lib().mtk_set_stream(self.dev.handle, self.handle))
+        return self
+
+    def __exit__(self, *exc):
+        mtk._check(mtk.lib().mtk_set_stream(self.dev.handle, None))
+
+    def close(self):
+        assert _hip().hipStreamSynchronize(self.handle) == 0 and _hip().hipStreamDestroy(self.handle) == 0
+
+
+class _Case:
+    """A plan on inputs of its own, an output buffer and the eager result on the context's own stream."""
+
+    def __init__(self, dev, case, seed):
+        self.dev, self.plan = dev, _plan(dev, case)
+        Q, K, V = _inputs(case, seed)
+        self.shape, self.bufs = Q.shape, [dev.upload(x) for x in (Q, K, V)] + [dev.empty(Q.nbytes)]
+        self.run()
+        dev.sync()
+        self.ref = self.read()
+
+    def run(self):
+        self.plan.run(*self.bufs)
+
+    def poison(self):
+        self.dev.upload_into(self.bufs[3], np.full(self.shape, 0x7E00, np.uint16))
+
+    def read(self):
+        return self.dev.download(self.bufs[3], self.shape, np.uint16).copy()
+
+    def close(self):
+        for b in self.bufs:
+            b.free()
+
+
+@pytest.mark.gpu
+def test_streams_and_captures_have_regions_of_their_own():
+    # more streams and captures than there are regions, all at work at once: every result is that of the
+    # context's own stream, also once the streams have gone and others take their regions
+    dev = mtk.Device(0)  # the captures' regions stay taken in a context
+    cases = [_Case(dev, SPLIT[i % len(SPLIT)], 300 + 10 * i) for i in range(20)]
+    hip = _hip()
+    for _ in range(2):
+        streams = [_Stream(dev) for _ in cases]
+        for c in cases:
+            c.poison()
+        for _ in range(3):
+            for c, st in zip(cases, streams):
+                with st:
+                    c.run()
+        for st in streams:
+            st.close()
+        assert all(np.array_equal(c.read(), c.ref) for c in cases)
+    st = _Stream(dev)
+    with st:
+        names = cases[0].plan.profile([cases[0].plan.args(*cases[0].bufs)], warmup=1, iters=2)["kernels"]
+    assert any("combine" in n for n in names), names  # the splits are shared out on an external stream too
+    graphs = []
+    try:
+        for c in cases:
+            g, e = ctypes.c_void_p(), ctypes.c_void_p()
+            with st:
+                assert hip.hipStreamBeginCapture(st.handle, 2) == 0  # relaxed
+                c.run()
+                c.run()
+                assert hip.hipStreamEndCapture(st.handle, ctypes.byref(g)) == 0
+            assert hip.hipGraphInstantiate(ctypes.byref(e), g, None, None, ctypes.c_size_t(0)) == 0
+            graphs.append((g, e))
+        others = [_Stream(dev) for _ in range(4)]
+        for _ in range(3):
+            for c in cases:
+                c.poison()
+            for i, (_, e) in enumerate(graphs):
+                assert hip.hipGraphLaunch(e, others[i % 4].handle) == 0
+            for o in others:
+                assert hip.hipStreamSynchronize(o.handle) == 0
+            assert all(np.array_equal(c.read(), c.ref) for c in cases)
+            for c in cases:  # eager calls between the replays
+                c.run()
+            dev.sync()
+        for o in others:
+            o.close()
+    finally:
+        for g, e in graphs:
+            hip.hipGraphExecDestroy(e)
+            hip.hipGraphDestroy(g)
+        st.close()
+        for c in cases:
+            c.close()
+        dev.close()
+
+
+@pytest.mark.gpu
+def test_two_threads_on_one_context(dev):
+    # kernels of two threads' calls on the context's own stream do not interleave on its partial sums
+    cases = [_Case(dev, SPLIT[i], 500 + 10 * i) for i in (0, 3)]
+    errors = []
+
+    def work(c):
+        try:
+            for _ in range(200):
+                c.run()
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+
+    for c in cases:
+        c.poison()
+    threads = [threading.Thread(target=work, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    dev.sync()
+    assert not errors, errors
+    for c in cases:
+        assert np.array_equal(c.read(), c.ref)
+        c.close()
+
+
+@pytest.mark.gpu
+def test_launches_do_not_allocate(dev):
+    # what a plan needs is there when it has been created: the first call of a new context takes no memory
+    hip = _hip()
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    own = mtk.Device(0)
+    try:
+        Q, K, V = _inputs(SPLIT[0])
+        bufs = [own.upload(x) for x in (Q, K, V)] + [own.empty(Q.nbytes)]
+        small = mtk.AttentionPlan(own, 1, 8, 1, 255, 128, H_kv=2)  # another kernel of the same code object first
+        small.run(*bufs)
+        plan = _plan(own, SPLIT[0])
+        own.sync()
+        before = free()
+        plan.run(*bufs)
+        own.sync()
+        assert free() == before
+        for b in bufs:
+            b.free()
+    finally:
+        own.close()
