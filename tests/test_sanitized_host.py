@@ -14,7 +14,7 @@ import example_matmul_metal4_amd as mtk
 
 #: files with tests of the planner alone
 PLANNED = ["test_abi", "test_attention_bwd_shared_gpu", "test_attention_kv_gpu", "test_attention_plan_sweep_gpu",
-           "test_attention_bwd_plan_sweep_gpu", "test_conv_plan_sweep_gpu", "test_conv_quarter_gpu", "test_gemm_plan_sweep_gpu",
+           "test_attention_bwd_plan_sweep_gpu", "test_causal_order_gpu", "test_conv_plan_sweep_gpu", "test_conv_quarter_gpu", "test_gemm_plan_sweep_gpu",
            "test_gemm_quarter_gpu", "test_gemm_tall_gpu"]
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
