@@ -288,3 +288,44 @@ def test_launches_do_not_allocate(dev):
             b.free()
     finally:
         own.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[3], CASES[10], SPLIT[0], SPLIT[1], SPLIT[3]], ids=str)
+def test_values_that_are_not_finite(dev, case):
+    # what is not finite reaches the rows and dims that read it and no others, and rows whose scores all lie
+    # far below any weight's range are still averaged
+    B, H, Hkv, Sq, Skv, D, causal, dtype = case
+    G = H // Hkv
+    Q, K, V = (oracle.to_f32(x, dtype) for x in _inputs(case, 640))
+    run = lambda q, k, v: mtk.attention(dev, *(oracle.from_f32(x, dtype) for x in (q, k, v)), causal=causal, dtype=dtype,
+                                        return_lse=True)
+    f = lambda x: oracle.to_f32(x, dtype)
+    O, lse = run(Q, K, V)
+    # a NaN and an infinity in one query row each: those rows only
+    q, rows = Q.copy(), [(0, Sq - 1, 0), (B - 1, Sq - 1, H - 1)]
+    q[rows[0]][D // 2], q[rows[1]][0] = np.nan, np.inf
+    o, l = run(q, K, V)
+    bad = np.zeros((B, Sq, H), bool)
+    for r in rows:
+        bad[r] = True
+    assert np.all(np.isnan(f(o))[bad]) and np.array_equal(o.view(np.uint16)[~bad], O.view(np.uint16)[~bad])
+    assert np.array_equal(l.transpose(0, 2, 1)[~bad], lse.transpose(0, 2, 1)[~bad])
+    # an infinity and a NaN in V at the last key: one dim each, of the rows that see it (the last queries) and of
+    # no row of another K/V head
+    v = V.copy()
+    v[0, Skv - 1, 0, 1], v[0, Skv - 1, 0, 3] = np.inf, np.nan
+    o = f(run(Q, K, v)[0])
+    assert not np.isfinite(o[0, Sq - 1, :G, 1]).any() and np.isnan(o[0, Sq - 1, :G, 3]).all()
+    other = np.ones(O.shape, bool)
+    other[0, :, :G, [1, 3]] = False
+    assert np.array_equal(o[other], f(O)[other])
+    # equal scores of about -2e7: every weight of a row is the same
+    q, k = np.zeros_like(Q), np.zeros_like(K)
+    q[..., 0], k[..., 0] = 6e4, -3750
+    o, _ = run(q, k, V)
+    exp = oracle.attention(*(oracle.from_f32(x, dtype) for x in (np.zeros_like(Q), k, V)), causal=causal, dtype=dtype)
+    # equal weights up to a rounding each (16 bits), and the output's
+    bound = oracle.ulp(exp, dtype) + 2 * (2.0 ** -11 if dtype == "f16" else 2.0 ** -8) * oracle.attention(
+        *(oracle.from_f32(x, dtype) for x in (np.zeros_like(Q), k, np.abs(V))), causal=causal, dtype=dtype)
+    assert np.all(np.abs(f(o) - exp) <= bound), np.abs(f(o) - exp).max()
