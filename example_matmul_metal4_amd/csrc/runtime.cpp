@@ -1161,21 +1161,32 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   //     tiles for 8 wavefronts)
   //   sequences of at most half a workgroup per CU: B 1, H 8, 1023 x 1023, D 128: 23.5 -> 12.7; 2048 x
   //     2048: 41 -> 35, causal 42 -> 24; but B 4, H 12, 512 x 512, D 64 (192 blocks): 11.9 against 16.6.
-  //     At D 128 one workgroup fits a CU: a second round of a few uncausal, short ones loses (B 3, H 16/4,
-  //     238 x 238, 360 workgroups: 10.5 against 14.4), as do D 64 (two per CU) and causal ones
-  //     (uneven anyway) below 512 keys (10 x 4 heads, 247 x 247, D 64: 8.0 against 9.3).
-  //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the
-  //     plan's choice (its kernel-select is fixed for such shapes; 4 x 1000 x 1000: 23 against 11).
+  //     One key-split workgroup fits a CU (its registers), and a second round of them has to be long enough.
+  //     From 21000 random calls timed on both, second rounds, 128-query time / key-split time (mean, lowest):
+  //     D 128 uncausal 8 to 31 key tiles 0.85 (0.70), from 32 on, the round at least half full, 1.13 (0.92);
+  //     D 128 causal, 16 to 23 tiles, at least half full 0.95 (0.87), less 1.14 (0.85), from 24 on 1.3 (1.03);
+  //     above D 128 uncausal 16 to 23 tiles 0.98 (0.94), from 24 on 1.2 (0.99); causal from 16 on 1.3 (1.04);
+  //     D 64 from 16 on 1.4 (0.92). Above D 128, where every row block takes two workgroups, third and
+  //     fourth rounds lose: 0.74 (0.51) (6 x 4 heads, 557 x 557, D 256: 30.0 against 55.7).
+  //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the choice
+  //     although the key-split ones are faster (400 random calls: 1.03x to 2.3x, mean 1.85x; 4 heads, 1000 x
+  //     1000: 23 against 11): that it is taken for small problems is a fixed part of kernel selection, on
+  //     which checks of the 128-query kernels at such sizes rely.
   //   fewer than 4 key tiles leave too many wavefronts without one (28 x 8 heads, 3 x 34: 5.4 against 5.8);
   //   K/V heads of their own gain only while the last round of workgroups is nearly full (19 x 16 heads,
-  //     1 x 1938: 304 workgroups, 60.0 against 66.3; B 32, H 32, 1 x 1024: 1024, 128 -> 99)
+  //     1 x 1938: 304 workgroups, 60.0 against 66.3; B 32, H 32, 1 x 1024: 1024, 128 -> 99), at D 128 with
+  //     more than 12 key tiles (12 x 32 heads, 1 x 370: 15.3 against 16.9)
   const int full = dp == 64 ? 2 : 4;  // 32-dim output blocks per workgroup, at most
   const int blocks32 = (d.D + 31) / 32;
   const long long wgs = units * ((blocks32 + full - 1) / full);
-  const bool full_rounds = wgs <= cus || d.H_kv < d.H || wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus);
+  const bool full_rounds = wgs <= cus || d.H_kv < d.H ||
+                           (wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus) && (dp != 128 || key_tiles > 12));
   const bool decode = d.S_q <= 16 && key_tiles >= 8 ? full_rounds : d.S_q <= 64 && wgs <= cus;
-  const bool one_round = wgs <= cus || (dp == 128 && !d.causal ? key_tiles >= 32 && wgs * 2 >= 3LL * cus : key_tiles >= 16);
-  const bool few = blocks * 2 <= cus && key_tiles >= 8 && one_round && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
+  const bool half = wgs * 2 >= 3LL * cus;  // the second round is at least half full
+  const bool second = wgs <= 2LL * cus && (dp == 128 && !d.causal ? key_tiles >= 32 && half
+                                           : dp == 128            ? key_tiles >= (half ? 24 : 16)
+                                                                  : key_tiles >= (dp == 256 && !d.causal ? 24 : 16));
+  const bool few = blocks * 2 <= cus && key_tiles >= 8 && (wgs <= cus || second) && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
   if (d.q_rows == 0 && !gen && !wide && key_tiles >= 4 && (decode || few)) {
     // fewer output blocks per workgroup while all workgroups still run at once: K is read again from
     // L2 by each, V once (B 1, H 32/8, 1 x 1024, D 128: 10.7 us with all four, 8.2 us with one)
