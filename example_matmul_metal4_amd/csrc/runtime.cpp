@@ -942,15 +942,21 @@ void set_divisor(D &out, int d) {
 //   more, where 128 columns are half empty (up to 64 output channels) and the walk is long: 658812 x 32, 64
 //     channels 3x3x3: 312 -> 279; 57138 x 32, 256 channels 3x3: 43.2 -> 42.5; with channels that are not a multiple
 //     of 64 (the 128x128 kernel decodes a tap per chunk) shorter ones too: 311808 x 16, 32 channels 3x3x3: 124
-//     -> 100; and up to three rounds of any width: 22960 x 72, 96 channels 5x5: 64.8 -> 38.6
+//     -> 100; and up to three rounds of any width: 22960 x 72, 96 channels 5x5: 64.8 -> 38.6. At two to four
+//     quarters per CU the 128x128 tiles still run at once and the walk has to be longer: of 700 random
+//     convolutions with up to 64 output channels, 128x128 time / quarter time, 512 to 768 quarters, channels in
+//     multiples of 64: 0.98 (0.89 to 1.1) for 20 to 27 K-tiles, 1.05 from 28, 1.15 from 50; 768 to 1024: 0.94, 0.98
+//     from 28, 1.03 from 50; more: 1.05, 1.13, 1.2. Other channels (8-wide loads), below 12 K-tiles: 0.99, 0.92 and
+//     1.03, from 12 on 1.1 to 1.7. 45738 x 64, 64 channels 5x5: 30.6 against 33.6
 //   otherwise the 128x128 tiles: 28749 x 512, 96 channels 3x3: 56.6 against 79.9
 //   one or two K-tiles: nothing to share (20400 x 256, 32 channels 1x1: 9.8 against 18.2)
-int conv_quarter(long long M, const mtk_conv_desc &d, int k_tiles, bool fast, int cus) {
+int conv_quarter(long long M, const mtk_conv_desc &d, int k_tiles, bool fast, int va, int cus) {
   if (d.C % 8 != 0 || d.KD > 10 || d.KH > 10 || d.KW > 10 || k_tiles < 3 || M >= (1 << 30)) return 0;
   const long long q = (M + 63) / 64 * ((d.O + 63) / 64);
   if (q <= cus) return 8;
   if (q <= 2LL * cus) return 4;
-  if (d.O <= 64 && k_tiles >= (fast ? 20 : 7)) return 4;
+  const int least = q > 4LL * cus ? (fast ? 20 : 7) : fast ? (q > 3LL * cus ? 50 : 28) : va == 8 ? 12 : 7;
+  if (d.O <= 64 && k_tiles >= least) return 4;
   return !fast && q <= 3LL * cus && k_tiles >= 12 ? 4 : 0;
 }
 
@@ -1065,7 +1071,7 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
   a.cOD = od;
   a.cOH = oh;
   a.cOW = ow;
-  const int quarter = conv_quarter(M, d, a.k_tiles, fast, ctx ? ctx->prop.multiProcessorCount : 256);
+  const int quarter = conv_quarter(M, d, a.k_tiles, fast, va, ctx ? ctx->prop.multiProcessorCount : 256);
   if (quarter) {
     g.name = std::string("mtk_conv_f16_gen_128x128_") + (!fast && va == 1 ? "v1q" : "q") + std::to_string(quarter);
     g.block = 64 * quarter;

@@ -65,3 +65,14 @@ def test_quarter_conv_in_the_middle_of_a_dword(dev):
         buf.free()
     assert got[0] == 0x1234 and got[-1] == 0x1234
     assert _bit_exact(dims, got[1:-1].view(np.float16).reshape(dims.y_shape()), x, w, b)
+
+
+def test_long_walks_between_two_and_four_quarters_per_cu():
+    # CPU: the planner alone. There the 128x128 tiles still run at once: quarters only for walks that are longer
+    def quarter(N, H, W, C, O, k):
+        dims = C2(N=N, H=H, W=W, C=C, O=O, KH=k, KW=k, PT=k // 2, PB=k // 2, PL=k // 2, PR=k // 2)
+        return _plan(None, 2, dims).describe().rsplit("_", 1)[1].endswith("q4")
+    for n, c, k, want in ((6, 64, 5, False), (6, 128, 5, True), (7, 64, 5, False), (7, 128, 5, True), (11, 64, 5, True),  # K-tiles
+                          (6, 16, 5, False), (6, 32, 5, True), (7, 72, 3, False), (7, 96, 3, True), (11, 56, 3, True)):
+        assert quarter(n, 80, 90, c, 64, k) == want, (n, c, k)
+    assert quarter(7, 80, 90, 72, 33, 3)  # output channels of odd count: the 128x128 kernel loads single elements
