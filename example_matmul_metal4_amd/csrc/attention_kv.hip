@@ -327,7 +327,9 @@ __device__ __forceinline__ void attn_kv(const mtk_attn_kargs &a) {
 }
 
 // The key splits' sums of every row, in split order. One thread per (row, 8 dims); a row's partials are
-// read once.
+// read once. The latency of these reads bounds it: 16 splits in flight and one wavefront per workgroup take
+// 4.9 us for 32 splits of 32 rows, D 128 (8 in flight, four wavefronts: 6.8), 4.0 for 16 (4.6); 32 in
+// flight spill (13.3).
 template <int DT>
 __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
   const int G = a.H / a.H_kv, rows = a.S_q * G, D = a.D, chunks = D / 8, S = a.kv_splits;
@@ -342,7 +344,7 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
   const float *ml = a.part_ml + 2 * pr0;
   const float *x = a.part + pr0 * a.part_ld + 8 * ch;
   KvSum total;
-  constexpr int kAhead = 8;  // splits whose partials are in flight at once
+  constexpr int kAhead = 16;  // splits whose partials are in flight at once
   for (int s0 = 0; s0 < S; s0 += kAhead) {
     KvSum t[kAhead];  // past the last split: no keys, which add nothing
 #pragma unroll
@@ -353,7 +355,11 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
         t[i] = KvSum{e.x, e.y, *(const f32x4 *)p, *(const f32x4 *)(p + 4)};
       }
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) add_keys(total, t[i]);
+    for (int i = 0; i < kAhead; i += 4) {  // few splits: no more than the last four are padding
+      if (s0 + i >= S) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) add_keys(total, t[i + j]);
+    }
   }
   const int q = rr / G;
   store_row<DT>(a, b, q, hk * G + (rr - q * G), 8 * ch, total, ch == 0);
@@ -363,10 +369,10 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
 
 using namespace mtk;
 
-extern "C" __global__ void __launch_bounds__(256) mtk_attn_kv_combine_f16(const mtk_attn_kargs a) {
+extern "C" __global__ void __launch_bounds__(64) mtk_attn_kv_combine_f16(const mtk_attn_kargs a) {
   attn_kv_combine<DT_F16>(a);
 }
-extern "C" __global__ void __launch_bounds__(256) mtk_attn_kv_combine_bf16(const mtk_attn_kargs a) {
+extern "C" __global__ void __launch_bounds__(64) mtk_attn_kv_combine_bf16(const mtk_attn_kargs a) {
   attn_kv_combine<DT_BF16>(a);
 }
 

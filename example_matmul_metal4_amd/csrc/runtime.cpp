@@ -1173,7 +1173,8 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   //     D 128 causal, 16 to 23 tiles, at least half full 0.95 (0.87), less 1.14 (0.85), from 24 on 1.3 (1.03);
   //     above D 128 uncausal 16 to 23 tiles 0.98 (0.94), from 24 on 1.2 (0.99); causal from 16 on 1.3 (1.04);
   //     D 64 from 16 on 1.4 (0.92). Above D 128, where every row block takes two workgroups, third and
-  //     fourth rounds lose: 0.74 (0.51) (6 x 4 heads, 557 x 557, D 256: 30.0 against 55.7).
+  //     fourth rounds lose: 0.74 (0.51) (6 x 4 heads, 557 x 557, D 256: 30.0 against 55.7), but for third
+  //     ones of causal self-attention without grouped heads: 1.07 (0.92) from 28 key tiles on.
   //     With fewer than 3/4 of a workgroup per CU below 1024 keys the 128-query kernel stays the choice
   //     although the key-split ones are faster (400 random calls: 1.03x to 2.3x, mean 1.85x; 4 heads, 1000 x
   //     1000: 23 against 11): that it is taken for small problems is a fixed part of kernel selection, on
@@ -1192,7 +1193,8 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   const bool second = wgs <= 2LL * cus && (dp == 128 && !d.causal ? key_tiles >= 32 && half
                                            : dp == 128            ? key_tiles >= (half ? 24 : 16)
                                                                   : key_tiles >= (dp == 256 && !d.causal ? 24 : 16));
-  const bool few = blocks * 2 <= cus && key_tiles >= 8 && (wgs <= cus || second) && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
+  const bool third = wgs <= 3LL * cus && dp == 256 && d.causal && d.H_kv == d.H && 4LL * d.S_q >= 3LL * d.S_kv && key_tiles >= 28;
+  const bool few = blocks * 2 <= cus && key_tiles >= 8 && (wgs <= cus || second || third) && (units * 4 >= 3LL * cus || d.S_kv >= 1024);
   if (d.q_rows == 0 && !gen && !wide && key_tiles >= 4 && (decode || few)) {
     // fewer output blocks per workgroup while all workgroups still run at once: K is read again from
     // L2 by each, V once (B 1, H 32/8, 1 x 1024, D 128: 10.7 us with all four, 8.2 us with one)
@@ -1243,8 +1245,8 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
       p->launches.push_back(kv_launch(full, true));
       Launch c = p->launches[0];
       c.name = std::string("mtk_attn_kv_combine_") + (d.dtype == MTK_F16 ? "f16" : "bf16");
-      c.block = 256;
-      c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 8) + 255) / 256);
+      c.block = 64;
+      c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 8) + 63) / 64);
       p->launches.push_back(c);
     } else {
       p->launches.push_back(kv_launch(ndb, false));

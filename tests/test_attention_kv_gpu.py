@@ -333,11 +333,12 @@ def test_values_that_are_not_finite(dev, case):
 
 def test_second_rounds_take_the_faster_kernel():
     # CPU: the planner alone. One key-split workgroup fits a CU: calls with a second round of them need long walks,
-    # and calls with more rounds, or short second ones, keep the 128-query kernel
+    # and most calls with more rounds, or short second ones, keep the 128-query kernel
     name = lambda *a, **kw: mtk.AttentionPlan(None, *a, **kw).describe().split("kernels: ")[1].split()[0]
     for a, kw, split in (
             ((6, 4, 557, 557, 256), {}, False), ((3, 2, 3700, 3700, 256), {}, False), ((1, 8, 1712, 2622, 256), dict(causal=True, H_kv=1), False),
-            ((1, 8, 1000, 1000, 256), dict(causal=True), True), ((1, 8, 1500, 1500, 256), dict(causal=True), False),
+            ((1, 8, 1000, 1000, 256), dict(causal=True), True), ((1, 8, 1500, 1500, 256), dict(causal=True), True), ((1, 8, 1500, 1500, 256), {}, False), ((1, 8, 1500, 1500, 256), dict(causal=True, H_kv=2), False),
+            ((1, 8, 1024, 1800, 256), dict(causal=True, H_kv=8), True), ((1, 8, 1200, 1800, 256), dict(causal=True), False), ((1, 8, 1800, 1800, 256), dict(causal=True), False),
             ((1, 8, 1024, 735, 256), {}, False), ((1, 8, 1024, 740, 256), {}, True), ((1, 8, 1024, 490, 256), dict(causal=True), True),
             ((4, 8, 490, 490, 128), dict(causal=True), False), ((4, 8, 512, 740, 128), dict(causal=True), True),
             ((3, 8, 480, 490, 128), dict(causal=True), True), ((3, 16, 238, 238, 128), dict(H_kv=4), False),
