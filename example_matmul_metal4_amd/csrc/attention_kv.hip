@@ -49,21 +49,27 @@ __device__ __forceinline__ f32x4 fma4(float f, f32x4 x, f32x4 y) {
 }
 __device__ __forceinline__ void add_keys(KvSum &s, const KvSum &t) {
 #pragma clang fp contract(off)
-  const float m = fmaxf(s.m, t.m), m0 = m == -INFINITY ? 0.0f : m;
-  const float f = __builtin_amdgcn_exp2f(s.m - m0), g = __builtin_amdgcn_exp2f(t.m - m0);
-  s.m = m;
+  const float d = t.m - s.m;  // NaN: no keys on either side
+  const float e = __builtin_amdgcn_exp2f(-fabsf(d));
+  const float f = d > 0.0f ? e : 1.0f, g = d > 0.0f ? 1.0f : d <= 0.0f ? e : 0.0f;
+  s.m = fmaxf(s.m, t.m);
   s.l = __builtin_fmaf(g, t.l, f * s.l);
   s.x0 = fma4(g, t.x0, f * s.x0);
   s.x1 = fma4(g, t.x1, f * s.x1);
 }
-// 8 dims of row (b, q, h) from d on, and the row's log-sum-exp if `lse`.
-template <int DT>
+// N (8 or 4) dims of row (b, q, h) from d on, and the row's log-sum-exp if `lse`.
+template <int DT, int N = 8>
 __device__ __forceinline__ void store_row(const mtk_attn_kargs &a, int b, int q, int h, int d, const KvSum &s, bool lse) {
   const float inv = s.l > 0.0f ? 1.0f / s.l : 0.0f;
-  if (d < a.D)
-    *(u32x4 *)((uint16_t *)a.O + (((size_t)b * a.S_q + q) * a.H + h) * a.D + d) =
-        u32x4{pack2<DT>(s.x0.x * inv, s.x0.y * inv), pack2<DT>(s.x0.z * inv, s.x0.w * inv),
-              pack2<DT>(s.x1.x * inv, s.x1.y * inv), pack2<DT>(s.x1.z * inv, s.x1.w * inv)};
+  if (d < a.D) {
+    uint16_t *o = (uint16_t *)a.O + (((size_t)b * a.S_q + q) * a.H + h) * a.D + d;
+    const u32x2 lo = {pack2<DT>(s.x0.x * inv, s.x0.y * inv), pack2<DT>(s.x0.z * inv, s.x0.w * inv)};
+    const u32x2 hi = {pack2<DT>(s.x1.x * inv, s.x1.y * inv), pack2<DT>(s.x1.z * inv, s.x1.w * inv)};
+    if constexpr (N == 8)
+      *(u32x4 *)o = u32x4{lo.x, lo.y, hi.x, hi.y};
+    else
+      *(u32x2 *)o = lo;
+  }
   if (lse) store_lse(a, b, h, q, 0, s.m, s.l);
 }
 
@@ -326,13 +332,13 @@ __device__ __forceinline__ void attn_kv(const mtk_attn_kargs &a) {
   }
 }
 
-// The key splits' sums of every row, in split order. One thread per (row, 8 dims); a row's partials are
-// read once. The latency of these reads bounds it: 16 splits in flight and one wavefront per workgroup take
-// 4.9 us for 32 splits of 32 rows, D 128 (8 in flight, four wavefronts: 6.8), 4.0 for 16 (4.6); 32 in
-// flight spill (13.3).
+// The key splits' sums of every row, in split order. One thread per (row, 4 dims); a row's partials are
+// read once. The latency of these reads and the additions of the one or two wavefronts of a row bound it.
+// 32 splits of 32 rows, D 128: 4.3 us with 16 splits in flight and one wavefront per workgroup (8 dims per thread:
+// 4.9, 8 splits and four wavefronts: 6.8), 16 splits: 3.8 (3.9, 4.6).
 template <int DT>
 __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
-  const int G = a.H / a.H_kv, rows = a.S_q * G, D = a.D, chunks = D / 8, S = a.kv_splits;
+  const int G = a.H / a.H_kv, rows = a.S_q * G, D = a.D, chunks = D / 4, S = a.kv_splits;
   const long long n = (long long)a.B * a.H_kv * rows * chunks;
   const long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (it >= n) return;
@@ -342,7 +348,7 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
   const int b = bh / a.H_kv, hk = bh - b * a.H_kv;
   const size_t pr0 = ((size_t)bh * a.q_blocks + rr / kKvRows) * S * kKvRows + rr % kKvRows;
   const float *ml = a.part_ml + 2 * pr0;
-  const float *x = a.part + pr0 * a.part_ld + 8 * ch;
+  const float *x = a.part + pr0 * a.part_ld + 4 * ch;
   KvSum total;
   constexpr int kAhead = 16;  // splits whose partials are in flight at once
   for (int s0 = 0; s0 < S; s0 += kAhead) {
@@ -351,8 +357,7 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
     for (int i = 0; i < kAhead; ++i)
       if (s0 + i < S) {
         const f32x2 e = *(const f32x2 *)(ml + (size_t)(s0 + i) * 2 * kKvRows);
-        const float *p = x + (size_t)(s0 + i) * kKvRows * a.part_ld;
-        t[i] = KvSum{e.x, e.y, *(const f32x4 *)p, *(const f32x4 *)(p + 4)};
+        t[i] = KvSum{e.x, e.y, *(const f32x4 *)(x + (size_t)(s0 + i) * kKvRows * a.part_ld)};
       }
 #pragma unroll
     for (int i = 0; i < kAhead; i += 4) {  // few splits: no more than the last four are padding
@@ -362,7 +367,7 @@ __device__ __forceinline__ void attn_kv_combine(const mtk_attn_kargs &a) {
     }
   }
   const int q = rr / G;
-  store_row<DT>(a, b, q, hk * G + (rr - q * G), 8 * ch, total, ch == 0);
+  store_row<DT, 4>(a, b, q, hk * G + (rr - q * G), 4 * ch, total, ch == 0);
 }
 
 }  // namespace mtk

@@ -1182,12 +1182,13 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   //   fewer than 4 key tiles leave too many wavefronts without one (28 x 8 heads, 3 x 34: 5.4 against 5.8);
   //   K/V heads of their own gain only while the last round of workgroups is nearly full (19 x 16 heads,
   //     1 x 1938: 304 workgroups, 60.0 against 66.3; B 32, H 32, 1 x 1024: 1024, 128 -> 99), at D 128 with
-  //     more than 12 key tiles (12 x 32 heads, 1 x 370: 15.3 against 16.9)
+  //     more than 12 key tiles (12 x 32 heads, 1 x 370, D 96: 15.3 against 16.9) or where the 256-query kernel
+  //     would run otherwise (25 x 16 heads, 1 x 225, D 128: 20.5 -> 15.7)
   const int full = dp == 64 ? 2 : 4;  // 32-dim output blocks per workgroup, at most
   const int blocks32 = (d.D + 31) / 32;
   const long long wgs = units * ((blocks32 + full - 1) / full);
   const bool full_rounds = wgs <= cus || d.H_kv < d.H ||
-                           (wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus) && (dp != 128 || key_tiles > 12));
+                           (wgs * 4 >= 3 * ((wgs + cus - 1) / cus * cus) && (dp != 128 || key_tiles > 12 || rows == 256));
   const bool decode = d.S_q <= 16 && key_tiles >= 8 ? full_rounds : d.S_q <= 64 && wgs <= cus;
   const bool half = wgs * 2 >= 3LL * cus;  // the second round is at least half full
   const bool second = wgs <= 2LL * cus && (dp == 128 && !d.causal ? key_tiles >= 32 && half
@@ -1246,7 +1247,7 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
       Launch c = p->launches[0];
       c.name = std::string("mtk_attn_kv_combine_") + (d.dtype == MTK_F16 ? "f16" : "bf16");
       c.block = 64;
-      c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 8) + 63) / 64);
+      c.grid = (unsigned)(((long long)d.B * d.H * d.S_q * (d.D / 4) + 63) / 64);
       p->launches.push_back(c);
     } else {
       p->launches.push_back(kv_launch(ndb, false));

@@ -335,12 +335,19 @@ def test_second_rounds_take_the_faster_kernel():
     # CPU: the planner alone. One key-split workgroup fits a CU: calls with a second round of them need long walks,
     # and most calls with more rounds, or short second ones, keep the 128-query kernel
     name = lambda *a, **kw: mtk.AttentionPlan(None, *a, **kw).describe().split("kernels: ")[1].split()[0]
+    causal, uncausal = dict(causal=True), {}
     for a, kw, split in (
-            ((6, 4, 557, 557, 256), {}, False), ((3, 2, 3700, 3700, 256), {}, False), ((1, 8, 1712, 2622, 256), dict(causal=True, H_kv=1), False),
-            ((1, 8, 1000, 1000, 256), dict(causal=True), True), ((1, 8, 1500, 1500, 256), dict(causal=True), True), ((1, 8, 1500, 1500, 256), {}, False), ((1, 8, 1500, 1500, 256), dict(causal=True, H_kv=2), False),
-            ((1, 8, 1024, 1800, 256), dict(causal=True, H_kv=8), True), ((1, 8, 1200, 1800, 256), dict(causal=True), False), ((1, 8, 1800, 1800, 256), dict(causal=True), False),
-            ((1, 8, 1024, 735, 256), {}, False), ((1, 8, 1024, 740, 256), {}, True), ((1, 8, 1024, 490, 256), dict(causal=True), True),
-            ((4, 8, 490, 490, 128), dict(causal=True), False), ((4, 8, 512, 740, 128), dict(causal=True), True),
-            ((3, 8, 480, 490, 128), dict(causal=True), True), ((3, 16, 238, 238, 128), dict(H_kv=4), False),
-            ((12, 32, 1, 370, 96), {}, False), ((12, 32, 1, 420, 96), {}, True), ((12, 32, 1, 370, 96), dict(H_kv=8), True)):
+            # above D 128
+            ((6, 4, 557, 557, 256), uncausal, False), ((3, 2, 3700, 3700, 256), uncausal, False),
+            ((1, 8, 1024, 735, 256), uncausal, False), ((1, 8, 1024, 740, 256), uncausal, True),
+            ((1, 8, 1000, 1000, 256), causal, True), ((1, 8, 1024, 490, 256), causal, True),
+            ((1, 8, 1500, 1500, 256), causal, True), ((1, 8, 1500, 1500, 256), uncausal, False),
+            ((1, 8, 1500, 1500, 256), dict(causal=True, H_kv=2), False), ((1, 8, 1200, 1800, 256), causal, False),
+            ((1, 8, 1800, 1800, 256), causal, False), ((1, 8, 1712, 2622, 256), dict(causal=True, H_kv=1), False),
+            # D 128
+            ((4, 8, 490, 490, 128), causal, False), ((4, 8, 512, 740, 128), causal, True),
+            ((3, 8, 480, 490, 128), causal, True), ((3, 16, 238, 238, 128), dict(H_kv=4), False),
+            ((12, 32, 1, 370, 96), uncausal, False), ((12, 32, 1, 420, 96), uncausal, True),
+            ((12, 32, 1, 370, 96), dict(H_kv=8), True), ((12, 32, 1, 370, 128), uncausal, True),
+            ((12, 32, 1, 370, 128), causal, False)):
         assert name(*a, **kw).startswith("mtk_attn_kv_") == split, (a, kw, name(*a, **kw))
