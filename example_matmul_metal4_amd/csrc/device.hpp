@@ -274,10 +274,11 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
 // pair, an XCD's last pairs started late and ran their longest blocks alone at the end.
 // Groups of 4 measured best (2 and 8: the same or slower; 16: 13 % slower).
 // With at most 4 pairs per XCD (and a workgroup for every CU: fewer end with the longest anyway) the
-// blocks of all pairs are dealt out longest first instead, by the hardware's own workgroup order (consecutive workgroups go to the XCDs in turn, so with a multiple
-// of 8 pairs each pair still stays on one XCD): a group's contiguous ids would span XCDs, its heavy
-// half on one and its light half on the next (dK/dV, shared walks, B 4, H 8/1, 976: 75 ->
-// 44 us; forward B 1, H 16/4, 4096, D 512: 1214 -> 852 us, H 12, D 64: 72.5 -> 67.7).
+// blocks of all pairs are dealt out longest first instead, by the hardware's own workgroup order
+// (consecutive workgroups go to the XCDs in turn, so with a multiple of 8 pairs each pair still stays
+// on one XCD): a group's contiguous ids would span XCDs, its heavy half on one and its light half on
+// the next (dK/dV, shared walks, B 4, H 8/1, 976: 75 -> 44 us; forward B 1, H 16/4, 4096, D 512:
+// 1214 -> 852 us, H 12, D 64: 72.5 -> 67.7).
 constexpr int kCausalGroup = 4;
 __device__ __forceinline__ void causal_order(int id, int nblk, int nbh, int &bh, int &rank) {
   if (nbh <= 8 * kCausalGroup && gridDim.x >= 256) {

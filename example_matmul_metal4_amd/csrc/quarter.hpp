@@ -5,8 +5,8 @@
 // latency per K-tile (about 1.5 us: 1023 cubed has 64 tiles of 16 K-tiles, 31 us for 2.1 GFLOP). Here
 //   * every wavefront takes every W-th K-tile of 64 for the whole 64x64 quarter (2 x 2 blocks of
 //     32x32x16 MFMAs: one fragment read per MFMA; 96x64: 3 x 2), staged global -> registers -> its own
-//     16 KB (20 KB) of LDS: no barrier until the end, and the loads of its next tile in flight meanwhile (two tiles ahead
-//     was slower: registers, 18.4 -> 19.5 us at 1024 x 1024 x 4096);
+//     16 KB (20 KB) of LDS: no barrier until the end, and the loads of its next tile in flight meanwhile
+//     (two tiles ahead was slower: registers, 18.4 -> 19.5 us at 1024 x 1024 x 4096);
 //   * the wavefronts' sums are parked in LDS and added in wavefront order, in fp32.
 // Operands stay as stored: rows along K are staged as in the tile kernels and read with 16-byte
 // fragment reads, K-major operands with transposed reads. ANY: rows at any 2-byte alignment.
@@ -26,7 +26,7 @@ struct QuarterOp {
   uint32_t step_k;    // bytes between K-tiles
 
   // Rows (columns) past the operand's end only reach outputs that are not stored; K past its end is
-  // zeroed by mask().
+  // zeroed by store().
   __device__ void init(int lane, int first, int ld, uint32_t mis) {
     const uint32_t row = (uint32_t)(KMAJOR ? lane >> 3 : first + (lane >> 3));
     const uint32_t col = (uint32_t)((KMAJOR ? first : 0) + 8 * (lane & 7));
