@@ -110,7 +110,11 @@ struct mtk_ctx {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     if (!parts) return -1;
-    if (hipStreamGetCaptureInfo(stream, &cs, &id) != hipSuccess || cs == hipStreamCaptureStatusInvalidated) return -1;
+    if (hipStreamGetCaptureInfo(stream, &cs, &id) != hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
+    if (cs == hipStreamCaptureStatusInvalidated) return -1;
     if (cs == hipStreamCaptureStatusNone) id = 0;
     if (stream == own_stream && !id) return 0;
     // No event is asked about or waited for that another stream has recorded: where that stream is being
@@ -1096,8 +1100,8 @@ int plan_conv(mtk_ctx *ctx, const mtk_conv_desc *d_in, mtk_plan **out) {
   p->bytes = (double)x_bytes + (double)w_bytes + 2.0 * (double)y_elems + (d.has_bias ? 2.0 * d.O : 0) +
              (oidhw ? 2.0 * (double)w_bytes : 0.0);  // the re-layout reads and writes the weights once
   char desc[288];
-  snprintf(desc, sizeof desc, "conv%dd f16 implicit-GEMM M=%lld N=%d K=%lld out=%dx%dx%d tile=%dx%d gather=%s grid=%u%s",
-           d.rank, M, d.O, K, od, oh, ow, quarter ? 64 : bm, quarter ? 64 : bn, quarter ? "gen" : kind, g.grid,
+  snprintf(desc, sizeof desc, "conv%dd f16 implicit-GEMM M=%lld N=%d K=%lld out=%dx%dx%d tile=%dx%d gather=%s%s grid=%u%s",
+           d.rank, M, d.O, K, od, oh, ow, quarter ? 64 : bm, quarter ? 64 : bn, kind, quarter ? "-quarter" : "", g.grid,
            oidhw ? " weights OIDHW (re-laid out in the workspace)" : "");
   p->description = desc;
   s = resolve(p);

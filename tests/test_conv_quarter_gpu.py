@@ -34,7 +34,7 @@ def test_which_plans_are_quartered():
     # CPU: the planner alone
     for rank, dims, kern in CASES:
         text = _plan(None, rank, dims).describe()
-        assert text.endswith("_" + kern) and " gather=gen " in text, (dims.as_dict(), text)
+        assert text.endswith("_" + kern) and "-quarter grid=" in text, (dims.as_dict(), text)
         _tile_and_grid(text, dims.N * dims.OD * dims.OH * dims.OW, dims.O, 64, 64)
     for dims in (C2(N=1, H=40, W=40, C=12, O=16), C2(N=1, H=40, W=40, C=16, O=16, KH=11, KW=3), C2(N=1, H=40, W=40, C=64, O=64, KH=1, KW=1),
                  C2(N=8, H=128, W=128, C=256, O=256), C2(N=4, H=100, W=100, C=96, O=256)):
@@ -76,3 +76,27 @@ def test_long_walks_between_two_and_four_quarters_per_cu():
                           (6, 16, 5, False), (6, 32, 5, True), (7, 72, 3, False), (7, 96, 3, True), (11, 56, 3, True)):
         assert quarter(n, 80, 90, c, 64, k) == want, (n, c, k)
     assert quarter(7, 80, 90, 72, 33, 3)  # output channels of odd count: the 128x128 kernel loads single elements
+
+
+# channels in multiples of 64 and too many quarters: the direct-to-LDS gather on 128x128 tiles, with filters of 36 and
+# 49 taps, strides, dilations, one-sided padding, three dimensions and remainders of both tile edges
+FAST = [(2, C2(N=2, H=100, W=101, C=64, O=96, KH=6, KW=6, PT=3, PB=2, PL=3, PR=2)),
+        (2, C2(N=2, H=100, W=101, C=64, O=70, KH=7, KW=7, PT=3, PB=3, PL=3, PR=3)),
+        (2, C2(N=8, H=131, W=133, C=128, O=40, SY=2, SX=2, DY=1, DX=2, PT=0, PB=1, PL=2, PR=1)),
+        (2, C2(N=3, H=61, W=97, C=192, O=202, KH=1, KW=5, SY=1, SX=1, PL=1, PR=3)),
+        (3, C3(N=1, D=12, H=41, W=43, C=64, O=130, KD=3, KH=2, KW=3, SZ=1, SY=1, SX=1, DZ=2, DY=1, DX=1, PF=2, PBk=1, PT=1, PB=0, PL=0, PR=2)),
+        (3, C3(N=2, D=15, H=60, W=62, C=64, O=66, SZ=2, SY=1, SX=2, DZ=1, DY=2, DX=1, PF=1, PBk=2, PT=1, PB=2, PL=1, PR=0))]
+
+
+def test_which_plans_keep_the_128x128_gather():
+    # CPU: the planner alone
+    for rank, dims in FAST:
+        assert _plan(None, rank, dims).describe().endswith("mtk_conv_f16_fast_128x128_d"), _plan(None, rank, dims).describe()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(FAST)))
+def test_128x128_gather(dev, case):
+    rank, dims = FAST[case]
+    x, w, b = gen.conv3d_activation(dims), gen.conv3d_weights(dims), gen.conv3d_bias(dims)
+    assert _bit_exact(dims, _run(dev, dims, x, w, b, rank=rank), x, w, b)
