@@ -19,7 +19,7 @@
 //     fp32, with each row's exponent offset and weight sum) a second kernel adds in split order. Where
 //     there is no buffer for them one workgroup walks the splits (the _seq kernels): the same bits.
 // With every CU reading, HBM bounds it: B 8, H 32, H_kv 8, 1 query, 4096 keys, D 128, bf16 (134 MB of
-// K and V): 105 us on the 128-query kernel -> 33 us (4.1 TB/s); 32 K/V heads (537 MB): 125 -> 98 us
+// K and V): 105 us on the 128-query kernel -> 31 us (4.3 TB/s); 32 K/V heads (537 MB): 125 -> 98 us
 // (5.5 TB/s, as a large copy). Short sequences are bound by the latency of a wavefront's tiles, about
 // 2 us each (1 x 8 heads x 1023, D 128: 23.6 -> 12.9 us, one tile in flight ahead of the current one).
 // Each wavefront stages its own key tiles global -> registers -> LDS (the next tile's loads are in

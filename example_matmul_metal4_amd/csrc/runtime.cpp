@@ -1168,7 +1168,7 @@ int plan_attn(mtk_ctx *ctx, const mtk_attn_desc *d_in, mtk_plan **out) {
   const int key_tiles = (d.S_kv + 31) / 32;
   // One box, us per call, 128-query kernel -> key-split kernels:
   //   few queries behind a cache (a 128-query block would be mostly padding, each query head reads the
-  //     cache again): B 8, H 32/8, 1 x 4096, D 128: 105 -> 33; B 1, H 32/8, 1 x 16384: 281 -> 19;
+  //     cache again): B 8, H 32/8, 1 x 4096, D 128: 105 -> 31; B 1, H 32/8, 1 x 16384: 281 -> 20;
   //     B 8, H 32/32, 1 x 4096: 125 -> 98 (5.5 TB/s); but 128 x 128, B 16, H 8: 9.3 against 12.1 (4 key
   //     tiles for 8 wavefronts)
   //   sequences of at most half a workgroup per CU: B 1, H 8, 1023 x 1023, D 128: 23.5 -> 12.7; 2048 x
