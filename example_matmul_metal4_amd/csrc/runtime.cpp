@@ -125,8 +125,10 @@ struct mtk_ctx {
       if (!id) {
         // A stream's first use creates the event; at a later one the handle may be another stream's by now,
         // the last one's work still running.
-        const hipError_t e = r.stream ? hipStreamWaitEvent(stream, r.done, 0) : hipEventCreateWithFlags(&r.done, hipEventDisableTiming);
+        const hipError_t e = r.stream ? hipStreamWaitEvent(stream, r.done, 0)
+                                      : hipEventCreateWithFlags(&r.done, hipEventDisableTiming);
         if (e != hipSuccess) {
+          if (!r.stream) r.done = nullptr;
           (void)hipGetLastError();
           return -1;
         }
@@ -529,10 +531,13 @@ int plan_gemm(mtk_ctx *ctx, const mtk_gemm_desc *d_in, mtk_plan **out) {
   // [K][M] with odd rows of B always, as no other kernel reads them: a requested tile, or partitions run
   // in sequence, is refused there.
   if (d.trans_a && !direct) {
-    const char *what = d.tile != 0 ? "a tile" : d.split_mode == MTK_SPLIT_SERIAL && split != 1 && k_tiles > 1 ? "in-workgroup split-K" : nullptr;
+    const char *what = d.tile != 0 ? "a tile"
+                       : d.split_mode == MTK_SPLIT_SERIAL && split != 1 && k_tiles > 1 ? "in-workgroup split-K"
+                                                                                       : nullptr;
     if (what) {
       delete p;
-      return fail(MTK_ERR_UNSUPPORTED, "A [K][M] with odd rows of B (ldb %d) runs on 64x64 workgroups: %s cannot be chosen", d.ldb, what);
+      return fail(MTK_ERR_UNSUPPORTED, "A [K][M] with odd rows of B (ldb %d) runs on 64x64 workgroups: %s cannot be chosen",
+                  d.ldb, what);
     }
   }
   Quarter quarter;
